@@ -281,8 +281,13 @@ int launch_merge(const AttnArgs& a, const AttnPlan& p, hipStream_t stream) {
 }
 
 template <typename T>
-int launch_generic(const AttnArgs& a, const AttnPlan& p, hipStream_t stream) {
+int launch_generic(const AttnArgs& a, const AttnPlan& p, int dtype, hipStream_t stream) {
   const dim3 grid(a.n_seq * a.hkv, p.tiles_max, p.parts_max);
+  if (attn_tiles_supported(a, dtype)) {
+    const int rc = launch_attn_tiles(a, p, dtype, stream);
+    if (rc != PKV_OK || p.parts_max == 1) return rc;
+    return launch_merge<T>(a, p, stream);
+  }
   if (a.d <= 64) {
     hipLaunchKernelGGL((attn_rows_kernel<T, 64>), grid, dim3(kThreads), 0, stream, a);
   } else if (a.d <= 128) {
@@ -410,12 +415,18 @@ AttnPlan plan_attention(int n_seq, int max_q_len, int hq, int hkv, int d,
     plen = 512;
     while (plen < 4096 && (int64_t)plen * 8 < kvb) plen *= 2;
   } else if (plen <= 0) {
-    // Aim for ~2048 workgroups so the 256 CUs stay busy even when most
-    // sequences are far below the bound.
-    int64_t parts_target = (2048 + units - 1) / (units > 0 ? units : 1);
+    // The tile kernel (head dim 32 / 64 / 128) splits a context only where
+    // its tiles leave CUs idle, into pieces of at least 512 tokens: its four
+    // wavefronts already share them, and the merge launch costs ~5 us (one
+    // prompt of 500 tokens 20 us split in two, 15 whole). The row kernel aims
+    // for ~2048 workgroups, so the 256 CUs stay busy even when most sequences
+    // are far below the bound.
+    const bool tiles = d == 32 || d == 64 || d == 128;
+    int64_t parts_target = ((tiles ? 256 : 2048) + units - 1) / (units > 0 ? units : 1);
     if (parts_target < 1) parts_target = 1;
     plen = (int)((kvb + parts_target - 1) / parts_target);
-    if (plen < 64) plen = 64;
+    const int least = tiles ? 512 : 64;
+    if (plen < least) plen = least;
   }
   plen = (plen + kChunk - 1) / kChunk * kChunk;
   p.part_tokens = plen;
@@ -507,9 +518,9 @@ int launch_attention(const AttnArgs& a, const AttnPlan& p, int dtype,
     return launch_decode_small(as, p, dtype, stream);
   }
   switch (dtype) {
-    case PKV_DTYPE_F32: return launch_generic<float>(a, p, stream);
-    case PKV_DTYPE_F16: return launch_generic<f16>(a, p, stream);
-    case PKV_DTYPE_BF16: return launch_generic<bf16>(a, p, stream);
+    case PKV_DTYPE_F32: return launch_generic<float>(a, p, dtype, stream);
+    case PKV_DTYPE_F16: return launch_generic<f16>(a, p, dtype, stream);
+    case PKV_DTYPE_BF16: return launch_generic<bf16>(a, p, dtype, stream);
   }
   return fail(PKV_ERR_INVALID, "unknown dtype %d", dtype);
 }

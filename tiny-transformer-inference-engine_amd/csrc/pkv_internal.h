@@ -326,6 +326,12 @@ __device__ __forceinline__ bool tile_geom(const AttnArgs& a, int s, int tile,
 bool decode_small_supported(int dtype, int max_q_len, int group, int d);
 int launch_decode_small(const AttnArgs& a, const AttnPlan& p, int dtype, hipStream_t stream);
 
+// attn_tiles.hip: tiles of kGenRows (query token, head) rows on the fp32
+// matrix cores, any group size, head dim 32 / 64 / 128; needs 16-byte aligned
+// pools, q and out.
+bool attn_tiles_supported(const AttnArgs& a, int dtype);
+int launch_attn_tiles(const AttnArgs& a, const AttnPlan& p, int dtype, hipStream_t stream);
+
 AttnPlan plan_attention(int n_seq, int max_q_len, int hq, int hkv, int d,
                         int max_blk, int block_size, int max_kv_len,
                         int part_tokens, int dtype);
