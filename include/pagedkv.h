@@ -58,6 +58,9 @@
  *   pkv_linear_rope_qkv_rmsnorm  attn_norm + q/k/v projections and RoPE
  *                                                    serving/paged_model.py:26-27,
  *                                                    models/rmsnorm.py:12-18, serving/paged_mqa.py:76-85
+ *   pkv_linear_tiles, pkv_linear_tiles_rope_qkv  the same projections for the rows
+ *                         of prompts (fp32)          serving/paged_mqa.py:76-85,112-113,
+ *                                                    models/mlp.py:24-32, serving/paged_model.py:20-29
  *   pkv_argmax_rows       greedy token choice: logits.argmax per sequence
  *   pkv_sample_rows       sample(): temperature, top-k, top-p, one draw per
  *                         row (sampling.py:94-137; the top-k step of
@@ -101,6 +104,11 @@ extern "C" {
 #define PKV_PART_PERSISTENT (-1)
 #define PKV_PART_STATIC (-2)
 #define PKV_PART_STREAM (-3)
+
+/* epilogue values of pkv_linear_tiles */
+#define PKV_EPILOGUE_NONE 0
+#define PKV_EPILOGUE_SWIGLU 1
+#define PKV_EPILOGUE_RESIDUAL 2
 
 #define PKV_OK 0
 #define PKV_ERR_INVALID (-1)     /* bad argument (shape, null pointer, ...) */
@@ -417,6 +425,36 @@ int pkv_linear_rope_qkv_rmsnorm(void* q_out, void* k_out, void* v_out, const voi
                                 const int32_t* positions, const float* cos_table,
                                 const float* sin_table, int max_pos, int hq, int hkv, int d,
                                 int dtype, int* status, void* stream);
+
+/*
+ * Projections of many fp32 rows (prefill): x [m, k] (rows x_stride elements
+ * apart), W [n, k] ([2n, k] = [gate rows; up rows] with PKV_EPILOGUE_SWIGLU),
+ * bias (nullable) one per weight row, out [m, n] contiguous:
+ *   PKV_EPILOGUE_NONE      out = x W^T + bias
+ *   PKV_EPILOGUE_SWIGLU    out = g * sigmoid(g) * u, as pkv_silu_mul of the
+ *                          gate and up halves
+ *   PKV_EPILOGUE_RESIDUAL  out += x W^T + bias
+ * Products and sums are fp32; the sum order is fixed and the same for every
+ * epilogue of one (m, weight rows, k). dtype must be PKV_DTYPE_F32, k a
+ * multiple of 32, x rows, W and out 16-byte aligned, x and W below 2 GiB
+ * (PKV_ERR_UNSUPPORTED otherwise). Replaces nn.Linear with the op that
+ * follows it for a prompt's rows (serving/paged_mqa.py:112-113,
+ * models/mlp.py:24-32, serving/paged_model.py:20-29).
+ */
+int pkv_linear_tiles(void* out, const void* x, const void* w, const void* bias, int64_t m,
+                     int64_t n, int64_t k, int64_t x_stride, int epilogue, int dtype,
+                     void* stream);
+
+/*
+ * pkv_linear_rope_qkv for many fp32 rows: the q/k/v projections as
+ * pkv_linear_tiles, q and k rotated as pkv_rope. Same requirements as
+ * pkv_linear_tiles. Replaces serving/paged_mqa.py:76-85 for a prompt's rows.
+ */
+int pkv_linear_tiles_rope_qkv(void* q_out, void* k_out, void* v_out, const void* x,
+                              const void* w_qkv, const void* bias, int64_t m, int64_t k,
+                              int64_t x_stride, const int32_t* positions,
+                              const float* cos_table, const float* sin_table, int max_pos, int hq,
+                              int hkv, int d, int dtype, int* status, void* stream);
 
 /*
  * Greedy token choice: ids[r] (int64) = the index of the largest of the

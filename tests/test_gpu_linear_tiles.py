@@ -1,0 +1,96 @@
+"""The fp32 many-row projections (csrc/linear_tiles.hip) at the edges of their
+tiles, against float64 products and the stand-alone RoPE / SwiGLU kernels.
+
+Tolerance: an fp32 sum of k products of N(0, 1) x N(0, 1/k) values errs by
+less than k 2^-24 max|partial sum| ~ 512 * 6e-8 * 4 = 1.2e-4 in the worst case
+and sqrt(k) of that in practice; 2e-5 is twice the practical figure."""
+import pytest
+import torch
+
+from serving import _native, fused_ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+TOL = dict(rtol=2e-5, atol=2e-5)
+
+
+def mk(seed, *shape, std=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(shape, generator=g, device=DEV) * std
+
+
+def tiles(x, w, bias, epilogue, out):
+    n = out.shape[1]
+    rc = _native.lib().pkv_linear_tiles(
+        out.data_ptr(), x.data_ptr(), w.data_ptr(), _native.ptr(bias), x.shape[0], n, x.shape[1],
+        x.stride(0), epilogue, 0, _native.stream_ptr(x.device))
+    _native.check(rc, "pkv_linear_tiles")
+    return out
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (63, 33, 64), (64, 64, 32), (65, 130, 96),
+                                   (300, 47, 512), (2146, 512, 512), (1025, 640, 128)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_plain_swiglu_residual(m, n, k, bias):
+    x = mk(1, m, k + 8)[:, :k]  # row stride past k
+    w = mk(2, 2 * n, k, std=k ** -0.5)
+    b = mk(3, 2 * n) if bias else None
+    want = x.double() @ w.double().t() + (b.double() if bias else 0)
+    full = tiles(x, w, b, _native.EPILOGUE_NONE, torch.empty(m, 2 * n, device=DEV))
+    torch.testing.assert_close(full.double(), want, **TOL)
+    # the epilogues are those of the same sums, bit for bit
+    sw = tiles(x, w, b, _native.EPILOGUE_SWIGLU, torch.empty(m, n, device=DEV))
+    assert torch.equal(sw, fused_ops.silu_mul(full[:, :n], full[:, n:]))
+    r = mk(4, m, 2 * n)
+    got = tiles(x, w, b, _native.EPILOGUE_RESIDUAL, r.clone())
+    assert torch.equal(got, r + full)
+
+
+@pytest.mark.parametrize("m,hq,hkv,d,k", [(65, 8, 1, 64, 512), (257, 4, 1, 32, 128),
+                                          (100, 3, 1, 10, 64), (1100, 8, 2, 64, 512)])
+def test_rope_qkv(m, hq, hkv, d, k):
+    x = mk(1, m, k)
+    w = mk(2, (hq + 2 * hkv) * d, k, std=k ** -0.5)
+    pos = torch.randint(0, 50, (m,), device=DEV, dtype=torch.int32)
+    pos[m // 2] = 77  # outside the tables: angle 0 and a status bit
+    ang = mk(3, 50, d // 2)
+    cos, sin = ang.cos().contiguous(), ang.sin().contiguous()
+    full = tiles(x, w, None, _native.EPILOGUE_NONE, torch.empty(m, w.shape[0], device=DEV))
+    nq, nk = hq * d, hkv * d
+    want = fused_ops.rope(full[:, :nq], full[:, nq:nq + nk], pos, cos, sin, v=full[:, nq + nk:],
+                          hq=hq, hkv=hkv, d=d)
+    got = [torch.empty_like(t) for t in want]
+    status = torch.zeros(1, dtype=torch.int32, device=DEV)
+    rc = _native.lib().pkv_linear_tiles_rope_qkv(
+        *(t.data_ptr() for t in got), x.data_ptr(), w.data_ptr(), None, m, k, k, pos.data_ptr(),
+        cos.data_ptr(), sin.data_ptr(), 50, hq, hkv, d, 0, status.data_ptr(),
+        _native.stream_ptr(x.device))
+    _native.check(rc, "pkv_linear_tiles_rope_qkv")
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert int(status.item()) == _native.PKV_STATUS_BAD_POS
+
+
+def test_wrappers_take_it_and_gradients_do_not(monkeypatch):
+    x, w = mk(1, 1100, 512), mk(2, 96, 512, std=512 ** -0.5)
+    calls = []
+    real = fused_ops._tiles
+    monkeypatch.setattr(fused_ops, "_tiles", lambda *a: calls.append(1) or real(*a))
+    y = fused_ops.linear(x, w)
+    assert calls
+    torch.testing.assert_close(y.double(), x.double() @ w.double().t(), **TOL)
+    wg = w.clone().requires_grad_()
+    fused_ops.linear(x, wg).sum().backward()
+    assert len(calls) == 1 and wg.grad is not None
+
+
+def test_refusals():
+    L = _native.lib()
+    x, w, out = mk(1, 64, 48), mk(2, 16, 48), torch.empty(64, 16, device=DEV)
+    st = _native.stream_ptr(x.device)
+    args = lambda k, epi, dt: (out.data_ptr(), x.data_ptr(), w.data_ptr(), None, 64, 16, k,  # noqa: E731
+                               48, epi, dt, st)
+    assert L.pkv_linear_tiles(*args(48, 0, 0)) == _native.PKV_ERR_UNSUPPORTED  # k % 32
+    assert L.pkv_linear_tiles(*args(32, 0, 2)) == _native.PKV_ERR_UNSUPPORTED  # bf16
+    assert L.pkv_linear_tiles(*args(32, 9, 0)) == _native.PKV_ERR_INVALID
+    assert L.pkv_linear_tiles(*args(64, 0, 0)) == _native.PKV_ERR_INVALID  # stride below k

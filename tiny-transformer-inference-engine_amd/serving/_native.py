@@ -47,6 +47,11 @@ PART_PERSISTENT = -1
 PART_STATIC = -2
 PART_STREAM = -3
 
+# epilogue values of pkv_linear_tiles
+EPILOGUE_NONE = 0
+EPILOGUE_SWIGLU = 1
+EPILOGUE_RESIDUAL = 2
+
 _lib = None
 _lock = threading.Lock()
 
@@ -104,6 +109,11 @@ _SIGNATURES = {
     "pkv_linear_rope_qkv_rmsnorm": ([_c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_float, _c_vp, _c_vp,
                                      _c_i64, _c_i64, _c_i64, _c_vp, _c_vp, _c_vp, _c_int, _c_int,
                                      _c_int, _c_int, _c_int, _c_vp, _c_vp], _c_int),
+    "pkv_linear_tiles": ([_c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_int,
+                          _c_int, _c_vp], _c_int),
+    "pkv_linear_tiles_rope_qkv": ([_c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_vp, _c_i64, _c_i64,
+                                   _c_i64, _c_vp, _c_vp, _c_vp, _c_int, _c_int, _c_int, _c_int,
+                                   _c_int, _c_vp, _c_vp], _c_int),
     "pkv_argmax_workspace_bytes": ([_c_i64, _c_i64, _c_int], _c_size),
     "pkv_argmax_rows": ([_c_vp, _c_vp, _c_i64, _c_i64, _c_i64, _c_int, _c_vp, _c_size, _c_vp],
                         _c_int),

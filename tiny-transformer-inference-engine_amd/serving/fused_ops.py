@@ -5,8 +5,9 @@ those ops fused into their epilogues (csrc/linear.hip); the greedy argmax
 (csrc/sampling.hip).
 
 Every function requires ROCm device tensors and the library (RuntimeError
-otherwise). The projections hand shapes their kernel does not take (fp32,
-k not a multiple of 32, more than LINEAR_MAX_ROWS rows or LINEAR_MAX_FEATURES
+otherwise). The projections hand fp32 prompts to the tile kernel
+(csrc/linear_tiles.hip, _tiles_ok) and other shapes their kernel does not take
+(k not a multiple of 32, more than LINEAR_MAX_ROWS rows or LINEAR_MAX_FEATURES
 features) to the library GEMM. Outputs are allocated with
 torch on the input's device and the current stream, so the calls can be
 captured in a HIP graph.
@@ -177,6 +178,41 @@ def _linear_ok(x2: torch.Tensor, w: torch.Tensor, bias, n_features: int) -> bool
             and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+# fp32 rows pkv_linear_tiles takes from the library GEMM. Sums of a layer's three
+# fused projections, library / tiles, us: at k = 512, 900 rows 40.3 / 41.9, 1300
+# 55.8 / 53.0, 2146 90.6 / 68.3, 4096 112 / 95; at k = 128, 257 rows 20.6 / 13.7; at
+# k = 1024, 2146 rows 223 / 209 but 4096 306 / 331
+TILES_MAX_K = 512
+TILES_SMALL_K = 256
+TILES_MIN_ROWS = 1024
+
+
+def _tiles_ok(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
+    """Whether pkv_linear_tiles takes this projection; calls that record
+    gradients stay on the framework's GEMM."""
+    ts = (x2, w) if bias is None else (x2, w, bias)
+    rows, k = x2.shape
+    return (x2.is_cuda and rows > (LINEAR_MAX_ROWS if k <= TILES_SMALL_K else TILES_MIN_ROWS)
+            and k <= TILES_MAX_K
+            and all(t.dtype == torch.float32 and t.device == x2.device for t in ts)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+            and (bias is None or bias.is_contiguous()) and w.is_contiguous()
+            and w.shape[1] == k and k % 32 == 0
+            and w.shape[0] <= LINEAR_MAX_FEATURES
+            and x2.stride(0) >= k and x2.stride(0) % 4 == 0
+            and rows * x2.stride(0) < 1 << 29 and w.numel() < 1 << 29
+            and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def _tiles(out, x2, w, bias, n, epilogue, what):
+    rc = _native.lib().pkv_linear_tiles(
+        out.data_ptr(), x2.data_ptr(), w.data_ptr(), _native.ptr(bias), x2.shape[0], n,
+        x2.shape[1], x2.stride(0), epilogue, _native.dtype_code(x2.dtype),
+        _native.stream_ptr(x2.device))
+    _native.check(rc, what)
+    return out
+
+
 def _x_stride(x2):
     return x2.stride(0) if x2.shape[0] > 1 else x2.shape[1]
 
@@ -187,6 +223,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     x2 = _as_rows(x)
     n = weight.shape[0]
     if not _linear_ok(x2, weight, bias, n):
+        if _tiles_ok(x2, weight, bias):
+            out = torch.empty((x2.shape[0], n), dtype=x.dtype, device=x.device)
+            _tiles(out, x2, weight, bias, n, _native.EPILOGUE_NONE, "linear")
+            return out.view(*x.shape[:-1], n)
         return F.linear(x, weight, bias)
     out = torch.empty((x2.shape[0], n), dtype=x.dtype, device=x.device)
     rc = _native.lib().pkv_linear(out.data_ptr(), x2.data_ptr(), weight.data_ptr(),
@@ -202,6 +242,10 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, b_gate_up: torch.Ten
     x2 = _as_rows(x)
     h = w_gate_up.shape[0] // 2
     if not _linear_ok(x2, w_gate_up, b_gate_up, 2 * h):
+        if w_gate_up.shape[0] == 2 * h and _tiles_ok(x2, w_gate_up, b_gate_up):
+            out = torch.empty((x2.shape[0], h), dtype=x.dtype, device=x.device)
+            _tiles(out, x2, w_gate_up, b_gate_up, h, _native.EPILOGUE_SWIGLU, "linear_swiglu")
+            return out.view(*x.shape[:-1], h)
         gu = F.linear(x, w_gate_up, b_gate_up)
         return silu_mul(gu[..., :h], gu[..., h:])
     _native.require_device(x2, w_gate_up, what="linear_swiglu")
@@ -223,7 +267,9 @@ def linear_rope_qkv(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: torch.Tensor | 
     x2 = _as_rows(x)
     T = x2.shape[0]
     nq, nk = hq * d, hkv * d
-    if not _linear_ok(x2, w_qkv, b_qkv, nq + 2 * nk):
+    few = _linear_ok(x2, w_qkv, b_qkv, nq + 2 * nk)
+    if not few and not (_tiles_ok(x2, w_qkv, b_qkv) and w_qkv.shape[0] == nq + 2 * nk
+                        and d % 2 == 0):
         qkv = F.linear(x2, w_qkv, b_qkv)
         return rope(qkv[:, :nq], qkv[:, nq:nq + nk], positions, cos, sin, v=qkv[:, nq + nk:],
                     hq=hq, hkv=hkv, d=d)
@@ -238,7 +284,8 @@ def linear_rope_qkv(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: torch.Tensor | 
     q = torch.empty((T, hq, d), dtype=x.dtype, device=x.device)
     k = torch.empty((T, hkv, d), dtype=x.dtype, device=x.device)
     v = torch.empty((T, hkv, d), dtype=x.dtype, device=x.device)
-    rc = _native.lib().pkv_linear_rope_qkv(
+    fn = _native.lib().pkv_linear_rope_qkv if few else _native.lib().pkv_linear_tiles_rope_qkv
+    rc = fn(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), x2.data_ptr(), w_qkv.data_ptr(),
         _native.ptr(b_qkv), T, x2.shape[1], _x_stride(x2), pos.data_ptr(), cos2.data_ptr(),
         sin2.data_ptr(), cos2.shape[0], hq, hkv, d, _native.dtype_code(x.dtype), None,
@@ -268,6 +315,12 @@ def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
     n = weight.shape[0]
     if (not _linear_ok(x2, weight, bias, n) or not resid.is_contiguous()
             or resid.dtype != x.dtype or resid.numel() != x2.shape[0] * n):
+        if (resid.is_contiguous() and resid.dtype == x.dtype and resid.device == x.device
+                and resid.numel() == x2.shape[0] * n and resid.data_ptr() % 16 == 0
+                and not (torch.is_grad_enabled() and resid.requires_grad)
+                and _tiles_ok(x2, weight, bias)):
+            return _tiles(resid, x2, weight, bias, n, _native.EPILOGUE_RESIDUAL,
+                          "linear_residual_")
         return resid.add_(linear(x, weight, bias).view(resid.shape))
     rc = _native.lib().pkv_linear_residual(
         resid.data_ptr(), x2.data_ptr(), weight.data_ptr(), _native.ptr(bias), x2.shape[0], n,
