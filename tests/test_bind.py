@@ -1,0 +1,33 @@
+"""The Python calls into the library (csrc/bind.cpp): every declared entry
+point, the C argument conversions, and errors reported on the same thread."""
+import pytest
+
+from serving import _native
+
+
+def test_every_entry_point_is_there():
+    calls = _native.calls()
+    for name in _native.EXPORTED:
+        if name != "pkv_last_error":  # read through lib() by check()
+            assert callable(getattr(calls, name)), name
+    assert calls.pkv_version() == _native.lib().pkv_version()
+
+
+def test_conversions():
+    calls = _native.calls()
+    args = (32, 1, 16, 1, 64, 64, 16, 0, 0, 2)
+    assert (calls.pkv_attention_workspace_bytes(*args)
+            == _native.lib().pkv_attention_workspace_bytes(*args) > 0)
+    with pytest.raises(TypeError):
+        calls.pkv_attention_workspace_bytes(*args[:-1])
+    with pytest.raises(TypeError):
+        calls.pkv_attention_workspace_bytes("32", *args[1:])
+    with pytest.raises(OverflowError):
+        calls.pkv_attention_workspace_bytes(1 << 40, *args[1:])
+
+
+def test_null_pointers_and_last_error():
+    rc = _native.calls().pkv_rms_norm(None, None, None, None, None, 1, 64, 64, 64, 1e-5, 2, None)
+    assert rc == _native.PKV_ERR_INVALID
+    with pytest.raises(ValueError, match="null"):
+        _native.check(rc, "pkv_rms_norm")

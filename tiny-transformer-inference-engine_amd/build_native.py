@@ -3,7 +3,8 @@
 Usage: python build_native.py [--jobs N]
 
 Every `csrc/*.hip` file is compiled to an object under `_build/` and linked
-into `lib/libpagedkv.so` next to this file. hipcc cross-compiles, so this runs
+into `lib/libpagedkv.so` next to this file; `csrc/bind.cpp` (the Python calls
+into it) becomes `lib/_pkvbind.so` with the host compiler. hipcc cross-compiles, so this runs
 on a machine without a GPU. Packed-FP32 instruction selection is switched off
 for the device code (`-packed-fp32-ops`).
 """
@@ -15,15 +16,18 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libpagedkv.so")
+BIND = os.path.join(LIBDIR, "_pkvbind.so")
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+CXX = os.environ.get("CXX", "g++")
 CFLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
@@ -76,6 +80,10 @@ def build(jobs: int = 4, verbose: bool = False) -> str:
     tmp = LIB + ".tmp"
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
     os.replace(tmp, LIB)
+    tmp = BIND + ".tmp"
+    _run([CXX, "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall",
+          "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "bind.cpp"), "-o", tmp])
+    os.replace(tmp, BIND)
     return LIB
 
 

@@ -8,6 +8,8 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -15,6 +17,7 @@ import torch
 
 _PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG_ROOT, "lib", "libpagedkv.so")
+BIND_PATH = os.path.join(_PKG_ROOT, "lib", "_pkvbind.so")
 
 DTYPE_CODES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 # OR-ed into a dtype code: the K/V pools hold fp8 e4m3 (torch.float8_e4m3fn)
@@ -53,6 +56,7 @@ EPILOGUE_SWIGLU = 1
 EPILOGUE_RESIDUAL = 2
 
 _lib = None
+_calls = None
 _lock = threading.Lock()
 
 _c_i64 = ctypes.c_int64
@@ -146,11 +150,35 @@ def lib():
     return _lib
 
 
+def calls():
+    """The library's entry points as the wrappers call them: the module
+    _pkvbind (csrc/bind.cpp), bound to lib()'s instance."""
+    global _calls
+    if _calls is not None:
+        return _calls
+    handle = lib()
+    with _lock:
+        if _calls is None:
+            if not os.path.exists(BIND_PATH):
+                raise RuntimeError(
+                    f"_pkvbind.so not found at {BIND_PATH}; build it with "
+                    "`python tiny-transformer-inference-engine_amd/build_native.py` "
+                    "(or __graft_entry__.build())")
+            loader = importlib.machinery.ExtensionFileLoader("_pkvbind", BIND_PATH)
+            spec = importlib.util.spec_from_file_location("_pkvbind", BIND_PATH, loader=loader)
+            mod = importlib.util.module_from_spec(spec)
+            loader.exec_module(mod)
+            mod.bind({name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value
+                      for name in _SIGNATURES})
+            _calls = mod
+    return _calls
+
+
 def is_available() -> bool:
     """True when the library loads and a ROCm device is visible."""
     try:
-        lib()
-    except (RuntimeError, OSError):
+        calls()
+    except (RuntimeError, OSError, ImportError):
         return False
     return torch.cuda.is_available()
 
@@ -191,8 +219,15 @@ def kv_code(q_dtype: torch.dtype, pool_dtype: torch.dtype) -> int:
     return dtype_code(q_dtype)
 
 
+# the current stream's handle by device index, without building a Stream object
+# (2.0 us against 0.1 a call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    if _raw_stream is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index)
 
 
 def ptr(t) -> int | None:

@@ -58,7 +58,7 @@ def _launch(q, k_pool, v_pool, block_tables, seq_lens, queryloc, n_seq,
     nb, bs, hkv, _ = k_pool.shape
     max_blk = block_tables.shape[1] if block_tables.dim() == 2 else 0
     code = _native.kv_code(q.dtype, k_pool.dtype)
-    L = _native.lib()
+    L = _native.calls()
     ws_bytes = L.pkv_attention_workspace_bytes(
         n_seq, max_q_len, hq, hkv, d, max_blk, bs, max_kv_len, part_tokens, code)
     ws = _native.current_workspace().get(q.device, ws_bytes)
@@ -235,7 +235,7 @@ def paged_attention_append_meta(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     if k.dtype != q.dtype:
         raise TypeError(f"new K/V rows ({k.dtype}) must have the queries' dtype ({q.dtype})")
     code = _native.kv_code(q.dtype, pool.dtype)
-    L = _native.lib()
+    L = _native.calls()
     max_blk = meta.block_tables.shape[1] if meta.block_tables.dim() == 2 else 0
     ws_bytes = L.pkv_attention_workspace_bytes(
         meta.num_seqs, meta.max_q_len, hq, pool.num_kv_heads, d, max_blk, pool.block_size,

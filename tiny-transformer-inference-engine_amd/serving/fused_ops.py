@@ -40,8 +40,8 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     if w.numel() != x.shape[-1]:
         raise ValueError(f"rms_norm: weight has {w.numel()} elements, rows have {x.shape[-1]}")
     x2, rows, stride = _rows(x, "rms_norm")
-    y = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    rc = _native.lib().pkv_rms_norm(
+    y = x.new_empty(x.shape)
+    rc = _native.calls().pkv_rms_norm(
         y.data_ptr(), None, x2.data_ptr(), None, w.data_ptr(), rows, x.shape[-1], stride,
         0, float(eps), _native.dtype_code(x.dtype), _native.stream_ptr(x.device))
     _native.check(rc, "rms_norm")
@@ -66,7 +66,7 @@ def add_rms_norm_(x: torch.Tensor, delta: torch.Tensor, weight: torch.Tensor,
         raise ValueError(f"add_rms_norm_: weight has {w.numel()} elements, rows have {dim}")
     d2, rows, dstride = _rows(delta, "add_rms_norm_")
     y = torch.empty_like(x)
-    rc = _native.lib().pkv_rms_norm(
+    rc = _native.calls().pkv_rms_norm(
         y.data_ptr(), x.data_ptr(), x.data_ptr(), d2.data_ptr(), w.data_ptr(), rows, dim, dim,
         dstride, float(eps), _native.dtype_code(x.dtype), _native.stream_ptr(x.device))
     _native.check(rc, "add_rms_norm_")
@@ -120,14 +120,14 @@ def rope(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor, cos: torch.T
     pos = pos.contiguous()
     qs, q_stride = _tok_rows(q, hq, d, "rope q")
     ks, k_stride = _tok_rows(k, hkv, d, "rope k")
-    q_out = torch.empty((T, hq, d), dtype=q.dtype, device=q.device)
-    k_out = torch.empty((T, hkv, d), dtype=q.dtype, device=q.device)
+    q_out = q.new_empty((T, hq, d))
+    k_out = q.new_empty((T, hkv, d))
     if v is not None:
         vs, v_stride = _tok_rows(v, hkv, d, "rope v")
-        v_out = torch.empty((T, hkv, d), dtype=q.dtype, device=q.device)
+        v_out = q.new_empty((T, hkv, d))
     else:
         vs, v_stride, v_out = None, 0, None
-    rc = _native.lib().pkv_rope(
+    rc = _native.calls().pkv_rope(
         q_out.data_ptr(), k_out.data_ptr(), _native.ptr(v_out), qs.data_ptr(), ks.data_ptr(),
         _native.ptr(vs), q_stride, k_stride, v_stride, pos.data_ptr(), cos2.data_ptr(),
         sin2.data_ptr(), cos2.shape[0], T, hq, hkv, d, _native.dtype_code(q.dtype), None,
@@ -146,8 +146,8 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     g2, rows, gs = _rows(gate, "silu_mul")
     u2, _, us = _rows(up, "silu_mul")
     cols = gate.shape[-1]
-    out = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
-    rc = _native.lib().pkv_silu_mul(out.data_ptr(), g2.data_ptr(), u2.data_ptr(), rows, cols,
+    out = gate.new_empty(gate.shape)
+    rc = _native.calls().pkv_silu_mul(out.data_ptr(), g2.data_ptr(), u2.data_ptr(), rows, cols,
                                     gs, us, _native.dtype_code(gate.dtype),
                                     _native.stream_ptr(gate.device))
     _native.check(rc, "silu_mul")
@@ -205,7 +205,7 @@ def _tiles_ok(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
 
 
 def _tiles(out, x2, w, bias, n, epilogue, what):
-    rc = _native.lib().pkv_linear_tiles(
+    rc = _native.calls().pkv_linear_tiles(
         out.data_ptr(), x2.data_ptr(), w.data_ptr(), _native.ptr(bias), x2.shape[0], n,
         x2.shape[1], x2.stride(0), epilogue, _native.dtype_code(x2.dtype),
         _native.stream_ptr(x2.device))
@@ -224,12 +224,12 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     n = weight.shape[0]
     if not _linear_ok(x2, weight, bias, n):
         if _tiles_ok(x2, weight, bias):
-            out = torch.empty((x2.shape[0], n), dtype=x.dtype, device=x.device)
+            out = x.new_empty((x2.shape[0], n))
             _tiles(out, x2, weight, bias, n, _native.EPILOGUE_NONE, "linear")
             return out.view(*x.shape[:-1], n)
         return F.linear(x, weight, bias)
-    out = torch.empty((x2.shape[0], n), dtype=x.dtype, device=x.device)
-    rc = _native.lib().pkv_linear(out.data_ptr(), x2.data_ptr(), weight.data_ptr(),
+    out = x.new_empty((x2.shape[0], n))
+    rc = _native.calls().pkv_linear(out.data_ptr(), x2.data_ptr(), weight.data_ptr(),
                                   _native.ptr(bias), x2.shape[0], n, x2.shape[1], _x_stride(x2),
                                   _native.dtype_code(x.dtype), _native.stream_ptr(x.device))
     _native.check(rc, "linear")
@@ -243,14 +243,14 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, b_gate_up: torch.Ten
     h = w_gate_up.shape[0] // 2
     if not _linear_ok(x2, w_gate_up, b_gate_up, 2 * h):
         if w_gate_up.shape[0] == 2 * h and _tiles_ok(x2, w_gate_up, b_gate_up):
-            out = torch.empty((x2.shape[0], h), dtype=x.dtype, device=x.device)
+            out = x.new_empty((x2.shape[0], h))
             _tiles(out, x2, w_gate_up, b_gate_up, h, _native.EPILOGUE_SWIGLU, "linear_swiglu")
             return out.view(*x.shape[:-1], h)
         gu = F.linear(x, w_gate_up, b_gate_up)
         return silu_mul(gu[..., :h], gu[..., h:])
     _native.require_device(x2, w_gate_up, what="linear_swiglu")
-    out = torch.empty((x2.shape[0], h), dtype=x.dtype, device=x.device)
-    rc = _native.lib().pkv_linear_swiglu(
+    out = x.new_empty((x2.shape[0], h))
+    rc = _native.calls().pkv_linear_swiglu(
         out.data_ptr(), x2.data_ptr(), w_gate_up.data_ptr(), _native.ptr(b_gate_up),
         x2.shape[0], h, x2.shape[1], _x_stride(x2), _native.dtype_code(x.dtype),
         _native.stream_ptr(x.device))
@@ -281,10 +281,10 @@ def linear_rope_qkv(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: torch.Tensor | 
     pos = pos.contiguous()
     if pos.numel() != T:
         raise ValueError("linear_rope_qkv: positions and x disagree on the token count")
-    q = torch.empty((T, hq, d), dtype=x.dtype, device=x.device)
-    k = torch.empty((T, hkv, d), dtype=x.dtype, device=x.device)
-    v = torch.empty((T, hkv, d), dtype=x.dtype, device=x.device)
-    fn = _native.lib().pkv_linear_rope_qkv if few else _native.lib().pkv_linear_tiles_rope_qkv
+    q = x.new_empty((T, hq, d))
+    k = x.new_empty((T, hkv, d))
+    v = x.new_empty((T, hkv, d))
+    fn = _native.calls().pkv_linear_rope_qkv if few else _native.calls().pkv_linear_tiles_rope_qkv
     rc = fn(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), x2.data_ptr(), w_qkv.data_ptr(),
         _native.ptr(b_qkv), T, x2.shape[1], _x_stride(x2), pos.data_ptr(), cos2.data_ptr(),
@@ -322,7 +322,7 @@ def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
             return _tiles(resid, x2, weight, bias, n, _native.EPILOGUE_RESIDUAL,
                           "linear_residual_")
         return resid.add_(linear(x, weight, bias).view(resid.shape))
-    rc = _native.lib().pkv_linear_residual(
+    rc = _native.calls().pkv_linear_residual(
         resid.data_ptr(), x2.data_ptr(), weight.data_ptr(), _native.ptr(bias), x2.shape[0], n,
         x2.shape[1], _x_stride(x2), _native.dtype_code(x.dtype), _native.stream_ptr(x.device))
     _native.check(rc, "linear_residual_")
@@ -338,8 +338,8 @@ def linear_swiglu_rmsnorm(x: torch.Tensor, norm_weight: torch.Tensor, eps: float
     if not (_linear_ok(x2, w_gate_up, b_gate_up, 2 * h) and _norm_ok(x2, norm_weight)):
         return linear_swiglu(rms_norm(x, norm_weight, eps), w_gate_up, b_gate_up)
     _native.require_device(x2, norm_weight, w_gate_up, what="linear_swiglu_rmsnorm")
-    out = torch.empty((x2.shape[0], h), dtype=x.dtype, device=x.device)
-    rc = _native.lib().pkv_linear_swiglu_rmsnorm(
+    out = x.new_empty((x2.shape[0], h))
+    rc = _native.calls().pkv_linear_swiglu_rmsnorm(
         out.data_ptr(), x2.data_ptr(), norm_weight.data_ptr(), float(eps), w_gate_up.data_ptr(),
         _native.ptr(b_gate_up), x2.shape[0], h, x2.shape[1], _x_stride(x2),
         _native.dtype_code(x.dtype), _native.stream_ptr(x.device))
@@ -369,10 +369,10 @@ def linear_rope_qkv_rmsnorm(x: torch.Tensor, norm_weight: torch.Tensor, eps: flo
     pos = pos.contiguous()
     if pos.numel() != T:
         raise ValueError("linear_rope_qkv_rmsnorm: positions and x disagree on the token count")
-    q = torch.empty((T, hq, d), dtype=x.dtype, device=x.device)
-    k = torch.empty((T, hkv, d), dtype=x.dtype, device=x.device)
-    v = torch.empty((T, hkv, d), dtype=x.dtype, device=x.device)
-    rc = _native.lib().pkv_linear_rope_qkv_rmsnorm(
+    q = x.new_empty((T, hq, d))
+    k = x.new_empty((T, hkv, d))
+    v = x.new_empty((T, hkv, d))
+    rc = _native.calls().pkv_linear_rope_qkv_rmsnorm(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), x2.data_ptr(), norm_weight.data_ptr(),
         float(eps), w_qkv.data_ptr(), _native.ptr(b_qkv), T, x2.shape[1], _x_stride(x2),
         pos.data_ptr(), cos2.data_ptr(), sin2.data_ptr(), cos2.shape[0], hq, hkv, d,
@@ -398,7 +398,7 @@ def argmax_rows(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.
         raise ValueError("argmax_rows: out must be a contiguous int64 tensor of rows elements")
     stride = lg.stride(0) if rows > 1 else vocab
     ws, wsb = _argmax_workspace(lg)
-    rc = _native.lib().pkv_argmax_rows(out.data_ptr(), lg.data_ptr(), rows, vocab, stride,
+    rc = _native.calls().pkv_argmax_rows(out.data_ptr(), lg.data_ptr(), rows, vocab, stride,
                                        _native.dtype_code(lg.dtype), _native.ptr(ws), wsb,
                                        _native.stream_ptr(logits.device))
     _native.check(rc, "argmax_rows")
@@ -409,7 +409,7 @@ def _argmax_workspace(lg):
     """The split-row argmax's counters and key words: the "argmax" slot of
     the current workspace (a graph step's own workspace under its scope)."""
     rows, vocab = lg.shape
-    wsb = int(_native.lib().pkv_argmax_workspace_bytes(rows, vocab, _native.dtype_code(lg.dtype)))
+    wsb = int(_native.calls().pkv_argmax_workspace_bytes(rows, vocab, _native.dtype_code(lg.dtype)))
     if wsb == 0:
         return None, 0
     return _native.current_workspace().get(lg.device, wsb, slot="argmax"), wsb
@@ -432,12 +432,22 @@ def sample_rows(logits: torch.Tensor, temperature: float, top_k: int, top_p: flo
     ids = torch.empty(rows, dtype=torch.long, device=logits.device)
     status = torch.zeros(1, dtype=torch.int32, device=logits.device)
     stride = lg.stride(0) if rows > 1 else vocab
-    rc = _native.lib().pkv_sample_rows(ids.data_ptr(), lg.data_ptr(), rows, vocab, stride,
+    rc = _native.calls().pkv_sample_rows(ids.data_ptr(), lg.data_ptr(), rows, vocab, stride,
                                        float(temperature), int(top_k), float(top_p),
                                        u.data_ptr(), _native.dtype_code(lg.dtype),
                                        status.data_ptr(), _native.stream_ptr(logits.device))
     _native.check(rc, "sample_rows")
     return ids, status
+
+
+def module_attr(mod: torch.nn.Module, name: str):
+    """mod.<name> for a parameter, buffer or submodule, read from its dict
+    where it is there: nn.Module's own lookup goes through a failed attribute
+    access first (0.25 us each, some thirty a layer)."""
+    for d in (mod._parameters, mod._modules, mod._buffers):
+        if name in d:
+            return d[name]
+    return getattr(mod, name)
 
 
 class FusedRows:
@@ -460,20 +470,21 @@ class FusedRows:
         off = 0
         base = self.weight.data_ptr()
         es = self.weight.element_size()
+        dev, dt = self.weight.device, self.weight.dtype
         for lin in self.linears:
-            w = lin.weight
-            if (w.device != self.weight.device or w.dtype != self.weight.dtype
+            w = module_attr(lin, "weight")
+            if (w.device != dev or w.dtype != dt
                     or w.data_ptr() != base + off * es or not w.is_contiguous()):
                 return False
             off += w.numel()
         if self.bias is not None:
             off, base, es = 0, self.bias.data_ptr(), self.bias.element_size()
             for lin in self.linears:
-                b = lin.bias
+                b = module_attr(lin, "bias")
                 if b is None or b.data_ptr() != base + off * es or b.dtype != self.bias.dtype:
                     return False
                 off += b.numel()
-        elif any(lin.bias is not None for lin in self.linears):
+        elif any(module_attr(lin, "bias") is not None for lin in self.linears):
             return False
         return True
 

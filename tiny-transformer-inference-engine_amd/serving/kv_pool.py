@@ -142,7 +142,7 @@ class KVPool:
         v = v.contiguous()
         slots = slot_mapping.contiguous()
         status = self._status()
-        rc = _native.lib().pkv_append(
+        rc = _native.calls().pkv_append(
             self.flat_k[layer].data_ptr(), self.flat_v[layer].data_ptr(), self.num_slots,
             k.data_ptr(), v.data_ptr(), slots.data_ptr(), k.shape[0],
             self.num_kv_heads * self.head_dim, _native.kv_code(k.dtype, self.dtype),
@@ -179,7 +179,7 @@ class KVPool:
         k = k.contiguous()
         v = v.contiguous()
         status = self._status()
-        rc = _native.lib().pkv_append_from_table(
+        rc = _native.calls().pkv_append_from_table(
             self.flat_k[layer].data_ptr(), self.flat_v[layer].data_ptr(), self.num_blocks,
             self.block_size, k.data_ptr(), v.data_ptr(), meta.block_tables.data_ptr(),
             meta.max_blocks, meta.query_start_loc.data_ptr(), meta.start_pos.data_ptr(),
@@ -206,7 +206,7 @@ class KVPool:
         k = torch.empty((seq_len, self.num_kv_heads, self.head_dim), dtype=self.dtype, device=self.device)
         v = torch.empty_like(k)
         status = self._status()
-        rc = _native.lib().pkv_gather(
+        rc = _native.calls().pkv_gather(
             k.data_ptr(), v.data_ptr(), self.kv[layer, 0].data_ptr(), self.kv[layer, 1].data_ptr(),
             self.num_blocks, self.block_size, bt.data_ptr(), bt.numel(), seq_len,
             self.num_kv_heads * self.head_dim, self._gather_code(),

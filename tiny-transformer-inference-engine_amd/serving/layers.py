@@ -46,11 +46,13 @@ class RoPE(nn.Module):
         lower precision holds its tables in that precision already (rounded
         once; rounding again changes nothing), so the fp32 copy is exact;
         it is cached until the buffers change."""
-        key = (self.cos.data_ptr(), self.cos._version, self.sin.data_ptr(), self.sin._version)
+        cos = fused_ops.module_attr(self, "cos")
+        sin = fused_ops.module_attr(self, "sin")
+        key = (cos.data_ptr(), cos._version, sin.data_ptr(), sin._version)
         if getattr(self, "_t32_key", None) != key:
             half = self.dim // 2
-            self._t32 = (self.cos.float().reshape(-1, half).contiguous(),
-                         self.sin.float().reshape(-1, half).contiguous())
+            self._t32 = (cos.float().reshape(-1, half).contiguous(),
+                         sin.float().reshape(-1, half).contiguous())
             self._t32_key = key
         return self._t32
 
@@ -126,8 +128,10 @@ class SwiGLU(nn.Module):
         the gate/up projection's prologue and the add in down_proj's
         epilogue (the same rounded values as the separate ops). Returns x."""
         w, b = self._gate_up.get()
-        h = fused_ops.linear_swiglu_rmsnorm(x, norm.weight, norm.eps, w, b)
-        return fused_ops.linear_residual_(x, h, self.down_proj.weight, self.down_proj.bias)
+        attr = fused_ops.module_attr
+        h = fused_ops.linear_swiglu_rmsnorm(x, attr(norm, "weight"), norm.eps, w, b)
+        down = attr(self, "down_proj")
+        return fused_ops.linear_residual_(x, h, attr(down, "weight"), attr(down, "bias"))
 
 
 class TokenEmbedding(nn.Module):

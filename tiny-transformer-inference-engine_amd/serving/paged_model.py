@@ -74,17 +74,19 @@ class PagedTransformer(nn.Module):
         The arithmetic is that of PagedBlock.forward_meta: each sum is
         rounded to the model dtype before it is normalised or carried on."""
         x = self.embedding(input_ids)
-        last = meta.query_start_loc[1:].long() - 1
         if not x.is_cuda:
             for layer in self.layers:
                 x = layer.forward_meta(x, pool, meta)
+            last = meta.query_start_loc[1:].long() - 1
             return self.lm_head(self.final_norm(x.index_select(0, last)))
         x = x.contiguous()
+        attr = fused_ops.module_attr
         for layer in self.layers:
-            layer.attn.forward_meta_residual_(x, layer.attn_norm, pool, layer.layer_idx, meta)
-            layer.mlp.forward_residual_(x, layer.mlp_norm)
+            attr(layer, "attn").forward_meta_residual_(x, attr(layer, "attn_norm"), pool,
+                                                       layer.layer_idx, meta)
+            attr(layer, "mlp").forward_residual_(x, attr(layer, "mlp_norm"))
         if not meta.is_decode:
-            x = x.index_select(0, last)
+            x = x.index_select(0, meta.query_start_loc[1:].long() - 1)
         return self.lm_head(self.final_norm(x))
 
 

@@ -109,10 +109,12 @@ class MQA_Paged(nn.Module):
         norm, layer and add). Returns x."""
         T, d_model = x.shape
         w, b = self._qkv.get()
-        cos, sin = self.rope._tables_fp32()
-        q, k, v = fused_ops.linear_rope_qkv_rmsnorm(x, norm.weight, norm.eps, w, b,
+        attr = fused_ops.module_attr
+        cos, sin = attr(self, "rope")._tables_fp32()
+        q, k, v = fused_ops.linear_rope_qkv_rmsnorm(x, attr(norm, "weight"), norm.eps, w, b,
                                                     meta.positions, cos, sin, self.num_heads,
                                                     self.num_kv_heads, self.headdim)
         out = paged_attention_append_meta(q, k, v, pool, layer_idx, meta)
-        return fused_ops.linear_residual_(x, out.view(T, d_model), self.out.weight,
-                                          self.out.bias)
+        proj = attr(self, "out")
+        return fused_ops.linear_residual_(x, out.view(T, d_model), attr(proj, "weight"),
+                                          attr(proj, "bias"))
