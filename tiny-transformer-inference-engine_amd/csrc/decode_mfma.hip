@@ -39,7 +39,7 @@ __global__ __launch_bounds__(kBlock, OCC) void decode_mfma_kernel(AttnArgs a) {
   using v8 = typename Ops<T>::v8;
   constexpr int G = 16 * NT;     // heads of the group
   constexpr int DT = D / 16;     // 16-wide column tiles of PV
-  constexpr int WAVE_BYTES = 2 * Geo::BYTES;
+  constexpr int WAVE_BYTES = Geo::BYTES;
   constexpr int OPITCH = D + 4;  // floats; +4 spreads head rows over banks
   constexpr int MERGE_BYTES = kWaves * G * OPITCH * 4;
   constexpr int MAIN_BYTES = kWaves * WAVE_BYTES;
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kBlock, OCC) void decode_mfma_kernel(AttnArgs a) {
   pv.bs_shift = a.bs_shift;
   ChunkCtx cx;
   cx.kl = lds + w * WAVE_BYTES;
-  cx.vl = cx.kl + Geo::BYTES;
+  cx.vl = cx.kl + Geo::KBYTES;
   cx.tbl = tbl;
   cx.prow = lane / Geo::CPR;
   cx.pcol = lane % Geo::CPR;

@@ -177,7 +177,7 @@ struct SkGeo {
   static constexpr int kWaves = NW;
   static constexpr int kBlock = 64 * kWaves;
   static constexpr int G = 16 * NT;
-  static constexpr int WAVE_BYTES = 2 * ChunkGeo<D>::BYTES;
+  static constexpr int WAVE_BYTES = ChunkGeo<D>::BYTES;
   template <typename S>
   using Combine = WaveCombine16<S, G, D, kWaves, kBlock>;
   static constexpr int MERGE_BYTES = kWaves * G * Combine<bf16>::OPITCH * 2;
@@ -298,7 +298,7 @@ __device__ __forceinline__ void decode_sk_body(AttnArgs a, SkArgs k, int wg,
   pv.bs_shift = a.bs_shift;
   ChunkCtx cx;
   cx.kl = lds + w * WAVE_BYTES;
-  cx.vl = cx.kl + Geo::BYTES;
+  cx.vl = cx.kl + Geo::KBYTES;
   cx.tbl = tbl;
   cx.prow = lane / Geo::CPR;
   cx.pcol = lane % Geo::CPR;

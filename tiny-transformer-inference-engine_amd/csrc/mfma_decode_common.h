@@ -155,19 +155,25 @@ __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_ex
 // LDS geometry of one 32-token chunk of K (or V) rows, D bf16/fp16 each.
 // Rows are padded by 16 bytes (PITCH = 2D + 16): row r starts 4r (mod 64)
 // banks further on for D = 128 (36r for D = 64), so the 16 rows an MFMA
-// fragment read touches at one 16-byte piece land on distinct bank groups,
-// and so do the 4 row groups of a V^T gather. Every fragment address is then
-// one base register plus an immediate offset.
+// fragment read touches at one 16-byte piece land on distinct bank groups.
+// V's rows are read by transposing reads, 32 bytes of each of 8 rows at once:
+// at D = 128 they are padded by 32 bytes, which puts the 8 on distinct banks
+// (by 16 bytes every bank was hit twice: 24 of 56 M LDS cycles of a long
+// prefill were conflicts); at D = 64 the 16 bytes already spread them. Every
+// fragment address is one base register plus an immediate offset.
 template <int D>
 struct ChunkGeo {
   static constexpr int CPR = D / 8;                 // 16-byte pieces per row
   static constexpr int ROW_BYTES = D * 2;
-  static constexpr int PITCH = ROW_BYTES + 16;
+  static constexpr int PITCH = ROW_BYTES + 16;                      // K rows
+  static constexpr int VPITCH = ROW_BYTES + (D == 128 ? 32 : 16);  // V rows
   static constexpr int ROWS_PER_LOAD = 64 / CPR;    // rows one wave load covers
   static constexpr int NPL = kChunk / ROWS_PER_LOAD;  // loads per lane per tensor
-  static constexpr int BYTES = kChunk * PITCH;
+  static constexpr int KBYTES = kChunk * PITCH;
+  static constexpr int BYTES = KBYTES + kChunk * VPITCH;  // K rows, then V rows
   static_assert(ROWS_PER_LOAD >= 1 && 64 % CPR == 0, "D must be 64 or 128");
   static __device__ __forceinline__ int off(int r, int c) { return r * PITCH + (c << 4); }
+  static __device__ __forceinline__ int voff(int r, int c) { return r * VPITCH + (c << 4); }
 };
 
 // K and V rows of one 32-token chunk held in registers between their loads
@@ -348,7 +354,7 @@ __device__ __forceinline__ void stage_new_row(const NewRow& nr, int cb, const Ch
       u32x4 x = *reinterpret_cast<const u32x4*>(nr.lds + lane * 16);
       if constexpr (KV8) x = widen8<T>(narrow8<T>(x));
       char* dst = lane < Geo::CPR ? cx.kl + Geo::off(r, lane)
-                                  : cx.vl + Geo::off(r, lane - Geo::CPR);
+                                  : cx.vl + Geo::voff(r, lane - Geo::CPR);
       *reinterpret_cast<u32x4*>(dst) = x;
     }
   }
@@ -384,7 +390,7 @@ __device__ __forceinline__ void stage_chunk(const ChunkRegs<NPL, KV8>& r, const 
       vp = ok ? vp : zero;
     }
     *reinterpret_cast<u32x4*>(cx.kl + Geo::off(row, cx.pcol)) = kp;
-    *reinterpret_cast<u32x4*>(cx.vl + Geo::off(row, cx.pcol)) = vp;
+    *reinterpret_cast<u32x4*>(cx.vl + Geo::voff(row, cx.pcol)) = vp;
   }
 }
 
@@ -455,17 +461,25 @@ __device__ __forceinline__ void chunk_update_sub(int c, const ChunkCtx& cx,
   bool move = false;
 #pragma unroll
   for (int nt = 0; nt < NC; ++nt) {
-    // token 16h + 4 grp + rr of the chunk is in range iff 16h + rr < lim
-    const int lim = seg_hi[nt] - cb - 4 * cx.grp;
-    float mx = -INFINITY;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        const float x = !MASK || 16 * h + rr < lim ? sacc[nt][h][rr] : -INFINITY;
-        sv[nt][4 * h + rr] = x;
-        mx = fmaxf(mx, x);
-      }
+      for (int rr = 0; rr < 4; ++rr) sv[nt][4 * h + rr] = sacc[nt][h][rr];
+    // uniform: the range ends inside the chunk (a mask on every chunk and the
+    // narrower V rows took 510 us on 4 prompts of 1-4 K tokens x 32 heads of
+    // 128; 484 without both)
+    if (MASK && cb + kChunk > seg_hi[nt]) {
+      // token 16h + 4 grp + rr of the chunk is in range iff 16h + rr < lim
+      const int lim = seg_hi[nt] - cb - 4 * cx.grp;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          if (16 * h + rr >= lim) sv[nt][4 * h + rr] = -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sv[nt][e]);
     move |= mx * sc > st.m[N0 + nt] + kLazy;  // also true on the first scores (m = -inf)
   }
   if (__builtin_amdgcn_ballot_w64(move) != 0) {
@@ -504,13 +518,13 @@ __device__ __forceinline__ void chunk_update_sub(int c, const ChunkCtx& cx,
   // and returns lane 4i + c the values c of source lanes i, 4 + i, 8 + i,
   // 12 + i; so source lane s addresses token row 4grp + s / 4 (and 16 rows
   // further for the second read), dims 16dt + 4 (s % 4) ... + 3.
-  const char* vt = cx.vl + (4 * cx.grp + (cx.l16 >> 2)) * Geo::PITCH + 8 * (cx.l16 & 3);
+  const char* vt = cx.vl + (4 * cx.grp + (cx.l16 >> 2)) * Geo::VPITCH + 8 * (cx.l16 & 3);
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) {
     const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (__attribute__((address_space(3))) v4s*)(vt + 32 * dt));
     const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) v4s*)(vt + 32 * dt + 16 * Geo::PITCH));
+        (__attribute__((address_space(3))) v4s*)(vt + 32 * dt + 16 * Geo::VPITCH));
     const v8s both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     v8 vf;
     __builtin_memcpy(&vf, &both, 16);

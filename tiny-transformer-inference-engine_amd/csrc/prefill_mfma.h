@@ -60,7 +60,7 @@ inline int64_t prefill_slots(int n_tokens, int n_seq, int group) {
 // accesses to different arrays never overlap).
 template <int D>
 struct PrefillLds {
-  static constexpr int kBufBytes = 2 * 2 * ChunkGeo<D>::BYTES;  // [stage][K | V], 16-aligned
+  static constexpr int kBufBytes = 2 * ChunkGeo<D>::BYTES;  // [stage][K | V], 16-aligned
   char* buf;
   int* tbl;      // kTblCap entries
   int* scan_sh;  // kPW
@@ -407,7 +407,7 @@ __device__ __forceinline__ void prefill_pair_body(AttnArgs a, int slot, int kvh,
     const int sa = min(X.lim[0], hi);
     const int cA = sa > lo ? (sa - lo + kChunk - 1) / kChunk : 0;
     auto step = [&](int c, Piece (&rg)[PER], unsigned& okm, auto both) {
-      char* kl = buf + (c & 1) * (2 * Geo::BYTES);
+      char* kl = buf + (c & 1) * Geo::BYTES;
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
         const bool ok = (okm >> k) & 1;
@@ -417,13 +417,14 @@ __device__ __forceinline__ void prefill_pair_body(AttnArgs a, int slot, int kvh,
           piece = widen8<T>(rg[k]);
         else
           piece = rg[k];
-        *reinterpret_cast<u32x4*>(kl + (is_v(k) ? Geo::BYTES : 0) + Geo::off(prow[k], pcol[k])) =
+        *reinterpret_cast<u32x4*>(kl + (is_v(k) ? Geo::KBYTES + Geo::voff(prow[k], pcol[k])
+                                                : Geo::off(prow[k], pcol[k]))) =
             ok ? piece : u32x4{0u, 0u, 0u, 0u};
       }
       issue(c + 2, rg, okm);
       __syncthreads();  // chunk c is staged; nobody reads the other buffer any more
       cx.kl = kl;
-      cx.vl = kl + Geo::BYTES;
+      cx.vl = kl + Geo::KBYTES;
       cx.seg_lo = lo;
       pair_chunk<T, D, decltype(both)::value>(X, c, lo, hi, cx);
       if (lo == 0 && c == 0 && dec) {  // its position has arrived: request the table entry
