@@ -84,6 +84,25 @@ def test_wrappers_take_it_and_gradients_do_not(monkeypatch):
     assert len(calls) == 1 and wg.grad is not None
 
 
+def test_transformed_calls_stay_with_the_framework():
+    """Autocast, forward-mode AD and torch.func see the projection as they see
+    F.linear; an x that is the residual itself is read before it is written."""
+    x, w, t = mk(1, 1100, 512), mk(2, 512, 512, std=512 ** -0.5), mk(3, 1100, 512)
+    with torch.no_grad():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert fused_ops.linear(x, w).dtype == torch.bfloat16
+        tangent = torch.func.jvp(lambda a: fused_ops.linear(a, w), (x,), (t,))[1]
+        torch.testing.assert_close(tangent.double(), t.double() @ w.double().t(), **TOL)
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(x, t)
+            out = torch.autograd.forward_ad.unpack_dual(fused_ops.linear(dual, w))
+        assert out.tangent is not None
+        both = torch.func.vmap(lambda a: fused_ops.linear(a, w))(torch.stack([x, t]))
+        torch.testing.assert_close(both[1], fused_ops.linear(t, w), **TOL)
+        want = x.double() + x.double() @ w.double().t()
+        torch.testing.assert_close(fused_ops.linear_residual_(x, x, w).double(), want, **TOL)
+
+
 def test_refusals():
     L = _native.lib()
     x, w, out = mk(1, 64, 48), mk(2, 16, 48), torch.empty(64, 16, device=DEV)

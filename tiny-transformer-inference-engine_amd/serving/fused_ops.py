@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _native
 
@@ -187,15 +188,24 @@ TILES_SMALL_K = 256
 TILES_MIN_ROWS = 1024
 
 
+def _transformed(ts) -> bool:
+    """Whether a call records, transforms or casts these tensors: gradients,
+    torch.func and forward-mode AD, autocast, tensor subclasses (tracing)."""
+    return ((torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+            or torch.is_autocast_enabled() or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in ts))
+
+
 def _tiles_ok(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
-    """Whether pkv_linear_tiles takes this projection; calls that record
-    gradients stay on the framework's GEMM."""
+    """Whether pkv_linear_tiles takes this projection; calls the
+    framework has to see stay on its GEMM."""
     ts = (x2, w) if bias is None else (x2, w, bias)
     rows, k = x2.shape
     return (x2.is_cuda and rows > (LINEAR_MAX_ROWS if k <= TILES_SMALL_K else TILES_MIN_ROWS)
             and k <= TILES_MAX_K
             and all(t.dtype == torch.float32 and t.device == x2.device for t in ts)
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+            and not _transformed(ts)
             and (bias is None or bias.is_contiguous()) and w.is_contiguous()
             and w.shape[1] == k and k % 32 == 0
             and w.shape[0] <= LINEAR_MAX_FEATURES
@@ -317,7 +327,9 @@ def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
             or resid.dtype != x.dtype or resid.numel() != x2.shape[0] * n):
         if (resid.is_contiguous() and resid.dtype == x.dtype and resid.device == x.device
                 and resid.numel() == x2.shape[0] * n and resid.data_ptr() % 16 == 0
-                and not (torch.is_grad_enabled() and resid.requires_grad)
+                and not _transformed((resid,))
+                # in place, and other workgroups still read x
+                and resid.untyped_storage().data_ptr() != x2.untyped_storage().data_ptr()
                 and _tiles_ok(x2, weight, bias)):
             return _tiles(resid, x2, weight, bias, n, _native.EPILOGUE_RESIDUAL,
                           "linear_residual_")
