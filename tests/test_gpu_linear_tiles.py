@@ -84,6 +84,16 @@ def test_wrappers_take_it_and_gradients_do_not(monkeypatch):
     assert len(calls) == 1 and wg.grad is not None
 
 
+@pytest.mark.parametrize("k", [32, 64, 96, 128, 160, 192, 224, 256, 1024])
+@pytest.mark.parametrize("m,n", [(257, 40), (4090, 250)])
+def test_slab_counts(k, m, n):
+    """Every remainder of the loop's rounds of four slabs, on the narrow and the
+    wide tiles. Tolerance: as above, for 1024 products sqrt(2) of 512's."""
+    x, w = mk(1, m, k), mk(2, n, k, std=k ** -0.5)
+    got = tiles(x, w, None, _native.EPILOGUE_NONE, torch.empty(m, n, device=DEV))
+    torch.testing.assert_close(got.double(), x.double() @ w.double().t(), rtol=3e-5, atol=3e-5)
+
+
 def test_transformed_calls_stay_with_the_framework():
     """Autocast, forward-mode AD and torch.func see the projection as they see
     F.linear; an x that is the residual itself is read before it is written."""

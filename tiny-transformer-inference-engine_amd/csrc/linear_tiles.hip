@@ -5,15 +5,21 @@
 //
 // What bounds it: the fp32 matrix pipe (155 TFLOP/s on this machine), which
 // vector instructions of the same SIMD do not overlap, and on few tiles the
-// barrier per slab. A workgroup owns 64 rows x 64 (or 32) weight rows; k is
-// walked in slabs of 32, loaded in whole 128-byte lines through buffer resources
-// whose scalar offset moves along k (no address arithmetic in the loop), staged
-// in two LDS buffers, one barrier a slab. (Operands loaded straight from memory
-// in matrix layout, without LDS, took 1.5 times as long: sixteen 16-byte pieces
-// of sixteen lines per instruction fill the L1. Slabs of 64 measured the same.)
-// Measured for a default prefill's layer (2146 rows, 512 wide), the library
-// GEMM with its separate element-wise kernel against this one, us: q/k/v + RoPE
-// 33.7 / 21.4, gate/up + SwiGLU 38.4 / 27.6, out + residual 18.5 / 19.3.
+// last, partly filled round of workgroups. A workgroup owns 64 rows x 64 (or 32)
+// weight rows; k is walked in slabs of 32, loaded in whole 128-byte lines
+// through buffer resources whose scalar offset moves along k (no address
+// arithmetic in the loop), four slabs ahead in registers, staged in two LDS
+// buffers, one barrier a slab. One slab ahead covered 512 to 1024 cycles of
+// matrix work against a longer round trip to memory: at 2146 rows x 1024 the
+// three fused forms took 191 us together, now 171; at 512 66 and 60. (Operands
+// loaded straight from memory in matrix layout, without LDS, took 1.5 times as
+// long: sixteen 16-byte pieces of sixteen lines per instruction fill the L1.
+// Slabs of 64, and LDS padding that bounds the workgroups per CU, measured the
+// same.)
+// Measured for a default prefill's layer (2146 rows, 512 wide), GPU time of the
+// library GEMM with its separate element-wise kernel against this one, us:
+// q/k/v + RoPE 33.4 / 19.2, gate/up + SwiGLU 37.7 / 26.4, out + residual 18.3 /
+// 17.2; 4096 rows x 1024 gate/up 134.8 / 138.3 (124 TFLOP/s), all three 311 / 302.
 #include "mfma_decode_common.h"
 
 namespace pkv {
@@ -47,6 +53,7 @@ struct TileArgs {
 };
 
 constexpr int kSlab = 32;          // k per staged slab
+constexpr int kAhead = 4;          // slabs in flight; even: slab s sits in LDS buffer s % 2
 constexpr int kSPitch = kSlab + 4;  // floats: 16 rows of one fragment read hit distinct banks
 
 template <int EPI, int XM>
@@ -92,17 +99,17 @@ __global__ __launch_bounds__(256, 3) void linear_tiles_kernel(TileArgs a) {
       const_cast<float*>(a.x), (short)0, -1, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(a.w), (short)0, -1, kRsrcWord3);
-  floatx4 g[NL];
-  auto fetch = [&](int slab) {
+  floatx4 g[kAhead][NL];  // the slabs in flight
+  auto fetch = [&](floatx4 (&r)[NL], int slab) {
 #pragma unroll
     for (int j = 0; j < NL; ++j)
-      g[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+      r[j] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
                                              32 * j < ROWS ? xr : wr, off[j], slab * 128, 0));
   };
-  auto stage = [&](int b) {
+  auto stage = [&](const floatx4 (&r)[NL], int b) {
 #pragma unroll
     for (int j = 0; j < NL; ++j)
-      *reinterpret_cast<floatx4*>(&lds[b][(tid / 8 + 32 * j) * kSPitch + 4 * (tid % 8)]) = g[j];
+      *reinterpret_cast<floatx4*>(&lds[b][(tid / 8 + 32 * j) * kSPitch + 4 * (tid % 8)]) = r[j];
   };
 
   floatx4 acc[2][XM];  // [weight tile][row tile]
@@ -111,13 +118,9 @@ __global__ __launch_bounds__(256, 3) void linear_tiles_kernel(TileArgs a) {
 #pragma unroll
     for (int t = 0; t < XM; ++t) acc[i][t] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int slabs = a.k / kSlab;
-  fetch(0);
-  stage(0);
-  fetch(min(1, slabs - 1));
-  __syncthreads();
-  for (int s = 0; s < slabs; ++s) {
-    const float* xl = &lds[s & 1][(16 * XM * wm + l16) * kSPitch + 4 * grp];
-    const float* wl = &lds[s & 1][(ROWS + 32 * wn + l16) * kSPitch + 4 * grp];
+  auto multiply = [&](int b) {
+    const float* xl = &lds[b][(16 * XM * wm + l16) * kSPitch + 4 * grp];
+    const float* wl = &lds[b][(ROWS + 32 * wn + l16) * kSPitch + 4 * grp];
     // product e of half h takes k = 16 h + 4 grp + e of every lane's row
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -136,11 +139,30 @@ __global__ __launch_bounds__(256, 3) void linear_tiles_kernel(TileArgs a) {
           for (int t = 0; t < XM; ++t)
             acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[i][e], xf[t][e], acc[i][t], 0, 0, 0);
     }
-    if (s + 1 < slabs) {
-      stage((s + 1) & 1);  // its readers passed the previous barrier
-      fetch(min(s + 2, slabs - 1));
+  };
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fetch(g[i], min(i, slabs - 1));
+  stage(g[0], 0);
+  __syncthreads();
+  // Whole rounds of kAhead slabs have no branch, which keeps the wait counts
+  // exact: slab s + 1 is waited for with kAhead - 2 younger ones in flight.
+  // Past the last slab its loads repeat, and what they stage is not read.
+  int s = 0;
+  for (; s + kAhead <= slabs; s += kAhead) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      fetch(g[i], min(s + i + kAhead, slabs - 1));
+      multiply(i & 1);
+      stage(g[(i + 1) % kAhead], (i + 1) & 1);  // its readers passed the previous barrier
       __syncthreads();
     }
+  }
+#pragma unroll
+  for (int i = 0; i < kAhead - 1; ++i) {
+    if (s + i >= slabs) break;
+    multiply(i & 1);
+    stage(g[i + 1], (i + 1) & 1);
+    __syncthreads();
   }
 
   // lane: rows m0 + 16 t + l16, features f0 + 16 i + 4 grp + 0..3 (swiglu:

@@ -156,8 +156,8 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 
 # the few-row projection kernels (csrc/linear.hip) take decode-sized row
-# counts; wider problems (prefill chunks, the vocabulary projection) and
-# fp32 go to the library GEMM
+# counts; fp32 prompts go to the tile kernel (_tiles_ok), other wider problems
+# (16-bit prefill chunks, the vocabulary projection) to the library GEMM
 LINEAR_MAX_ROWS = 256
 LINEAR_MAX_FEATURES = 16384
 
@@ -180,11 +180,11 @@ def _linear_ok(x2: torch.Tensor, w: torch.Tensor, bias, n_features: int) -> bool
 
 
 # fp32 rows pkv_linear_tiles takes from the library GEMM. Sums of a layer's three
-# fused projections, library / tiles, us: at k = 512, 900 rows 40.3 / 41.9, 1300
-# 55.8 / 53.0, 2146 90.6 / 68.3, 4096 112 / 95; at k = 128, 257 rows 20.6 / 13.7; at
-# k = 1024, 2146 rows 223 / 209 but 4096 306 / 331
-TILES_MAX_K = 512
-TILES_SMALL_K = 256
+# fused projections, library / tiles, us of GPU time: at k = 512, 300 rows 28.8 /
+# 27.6, 900 40.1 / 39.0, 2146 89 / 63, 4096 111 / 92; at k = 1024, 600 rows 67 / 82,
+# 1300 137 / 121, 2146 222 / 189, 4096 311 / 302; at k = 128, 300 rows 20.2 / 13.7
+TILES_MAX_K = 1024
+TILES_SMALL_K = 512
 TILES_MIN_ROWS = 1024
 
 
