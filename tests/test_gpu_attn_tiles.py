@@ -78,8 +78,47 @@ def test_many_tiles(dtype, causal):
 
 @pytest.mark.parametrize("bs", [8, 16])
 def test_table_windows_and_split(bs):
-    # contexts past one table window (255 blocks) and split over workgroups
+    # contexts split over workgroups in 512-token partitions, each inside one
+    # table window (255 blocks)
     check(problem([3, 1], [4200, 2037], 8, 1, 64, bs, torch.float32), torch.float32)
+
+
+@pytest.mark.parametrize("hq,d,bs,ctx", [(8, 32, 16, 4200), (8, 64, 8, 2100), (3, 128, 8, 4100),
+                                         (8, 64, 4, 1100), (5, 32, 2, 1100), (8, 64, 1, 700),
+                                         (8, 32, 1, 270), (8, 128, 2, 511)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_partition_across_table_windows(hq, d, bs, ctx, causal):
+    # one workgroup's keys cross the end of a window of 255 blocks, once to
+    # three times: every key counts once
+    p = problem([4, 21], [ctx - 4, ctx - 37], hq, 1, d, bs, torch.float32)
+    out = torch.empty_like(p["q"])
+    lse = torch.empty(out.shape[:2], device=DEV)
+    rc = _native.lib().pkv_paged_attention(
+        out.data_ptr(), lse.data_ptr(), p["q"].data_ptr(), p["k"].data_ptr(), p["v"].data_ptr(),
+        p["k"].shape[0], bs, p["table"].data_ptr(), p["table"].shape[1], p["lens"].data_ptr(),
+        p["qsl"].data_ptr(), 2, 25, 21, 0, hq, 1, d, 0.0, int(causal), 8192, 0, None, 0, None,
+        _native.stream_ptr(p["q"].device))
+    _native.check(rc, "pkv_paged_attention")
+    want, wl = ref.paged_attention(np64(p["q"]), np64(p["k"]), np64(p["v"]),
+                                   p["table"].cpu().numpy(), p["lens"].cpu().numpy(),
+                                   p["qsl"].cpu().numpy(), causal=causal)
+    np.testing.assert_allclose(np64(out), want, rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(lse.cpu().numpy(), wl, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_long_prompt_of_small_blocks(dtype):
+    # one prompt with enough tiles for a single partition, past a window's end:
+    # its last rows against the oracle (their queries alone see the same keys)
+    n, last = 2100, 70
+    p = problem([n], [0], 8, 1, 64, 8, dtype)
+    out, lse = paged_attn_fwd(p["q"], p["k"], p["v"], p["table"], p["lens"], p["qsl"], n)
+    want, wl = ref.paged_attention(np64(p["q"])[n - last:], np64(p["k"]), np64(p["v"]),
+                                   p["table"].cpu().numpy(), p["lens"].cpu().numpy(),
+                                   np.array([0, last], dtype=np.int32))
+    np.testing.assert_allclose(np64(out)[n - last:], want, atol=ATOL[dtype],
+                               rtol=1e-5 if dtype == torch.float32 else 0)
+    np.testing.assert_allclose(lse.cpu().numpy()[n - last:], wl, rtol=1e-5, atol=1e-5)
 
 
 def test_packed_grid():

@@ -48,7 +48,7 @@ static_assert(kTBlock == kTblCap, "one table entry per thread and window");
 
 template <int D>
 struct TileGeo {
-  static constexpr int C = D == 32 ? 32 : D == 64 ? 16 : 16;  // tokens per chunk
+  static constexpr int C = D == 32 ? 32 : 16;   // tokens per chunk
   static constexpr int HT = C / 16;             // 16-token MFMA tiles
   static constexpr int KP = D / 32;             // 32-dim step pairs
   static constexpr int DT = D / 16;             // 16-dim output tiles
@@ -147,8 +147,14 @@ __device__ __forceinline__ bool tile_chunks(const AttnArgs& a, const int32_t* __
   bool bad_block = false;
 
   // kTblCap - 1 blocks of tokens per window: one that starts inside a block
-  // still touches at most kTblCap table entries
-  const int win = (kTblCap - 1) << a.bs_shift;
+  // still touches at most kTblCap table entries. In whole chunks, so that a
+  // chunk reaches past its window's end only where that is kv_hi: scores are
+  // masked from lim (<= kv_hi) on, and a chunk across an inner window end would
+  // leave the next window's tokens in twice (block sizes below 16, and 32-token
+  // chunks with blocks of 16). Blocks past 2^20 tokens take smaller windows.
+  const int win = ((kTblCap - 1) << min(a.bs_shift, 20)) & ~(C - 1);
+  static_assert((C & (C - 1)) == 0 && C < kTblCap && kChunk % C == 0,
+                "windows and partitions start at whole chunks");
   for (int lo = kv_lo; lo < kv_hi; lo += win) {
     const int hi = min(lo + win, kv_hi);
     const int blk_lo = lo >> a.bs_shift;
@@ -158,7 +164,8 @@ __device__ __forceinline__ bool tile_chunks(const AttnArgs& a, const int32_t* __
     __syncthreads();
     const int nch = (hi - lo + C - 1) / C;
 
-    // Rows past hi re-read the window's last row (their scores are masked);
+    // Rows past hi re-read the window's last row (hi is kv_hi then, see win:
+    // their scores are masked);
     // rows whose table entry is outside the pool read block 0 and are zeroed
     // before use. off: byte offset of position pos's row.
     auto row_off = [&](int pos, bool& ok) {
