@@ -113,6 +113,34 @@ def test_transformed_calls_stay_with_the_framework():
         torch.testing.assert_close(fused_ops.linear_residual_(x, x, w).double(), want, **TOL)
 
 
+@pytest.mark.parametrize("shape", [(1,), (96,), (300, 96), (1, 96)])
+def test_bias_forms_of_the_framework(shape):
+    """A bias of one value per feature is the kernel's; one that broadcasts is
+    added as F.linear adds it. F.linear's sums differ by rounding only."""
+    x, w, b = mk(1, 300, 128), mk(2, 96, 128, std=128 ** -0.5), mk(3, *shape)
+    want = x.double() @ w.double().t() + b.double()
+    with torch.no_grad():
+        torch.testing.assert_close(fused_ops.linear(x, w, b).double(), want, **TOL)
+        r = mk(4, 300, 96)
+        got = fused_ops.linear_residual_(r.clone(), x, w, b)
+        torch.testing.assert_close(got.double(), r.double() + want, **TOL)
+        # products of two such sums of up to ~5 in size: 5 times their tolerance
+        gate, up = want[:, :48], want[:, 48:]
+        torch.testing.assert_close(fused_ops.linear_swiglu(x, w, b).double(),
+                                   torch.nn.functional.silu(gate) * up, rtol=1e-4, atol=1e-4)
+        pos = torch.zeros(300, dtype=torch.int32, device=DEV)  # angle 0: no rotation
+        cos, sin = torch.ones(4, 16, device=DEV), torch.zeros(4, 16, device=DEV)
+        q, k, v = fused_ops.linear_rope_qkv(x, w, b, pos, cos, sin, 1, 1, 32)
+        torch.testing.assert_close(torch.cat([q, k, v], 1).view(300, 96).double(), want, **TOL)
+
+
+@pytest.mark.parametrize("features", [95, 97])
+def test_wrong_bias_is_an_error(features):
+    x, w = mk(1, 300, 128), mk(2, 96, 128)
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        fused_ops.linear(x, w, mk(3, features))
+
+
 def test_refusals():
     L = _native.lib()
     x, w, out = mk(1, 64, 48), mk(2, 16, 48), torch.empty(64, 16, device=DEV)

@@ -197,21 +197,27 @@ def _transformed(ts) -> bool:
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in ts))
 
 
-def _tiles_ok(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
-    """Whether pkv_linear_tiles takes this projection; calls the
-    framework has to see stay on its GEMM."""
+def _tiles_fit(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
+    """Whether pkv_linear_tiles takes a projection of these operands; calls the
+    framework has to see stay on its GEMM, and so does a bias of any other shape
+    than one value per weight row, which is all the kernel reads."""
     ts = (x2, w) if bias is None else (x2, w, bias)
     rows, k = x2.shape
-    return (x2.is_cuda and rows > (LINEAR_MAX_ROWS if k <= TILES_SMALL_K else TILES_MIN_ROWS)
+    return (rows > (LINEAR_MAX_ROWS if k <= TILES_SMALL_K else TILES_MIN_ROWS)
             and k <= TILES_MAX_K
             and all(t.dtype == torch.float32 and t.device == x2.device for t in ts)
             and not _transformed(ts)
-            and (bias is None or bias.is_contiguous()) and w.is_contiguous()
+            and (bias is None or (bias.shape == w.shape[:1] and bias.is_contiguous()))
+            and w.is_contiguous()
             and w.shape[1] == k and k % 32 == 0
             and w.shape[0] <= LINEAR_MAX_FEATURES
             and x2.stride(0) >= k and x2.stride(0) % 4 == 0
             and rows * x2.stride(0) < 1 << 29 and w.numel() < 1 << 29
             and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def _tiles_ok(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
+    return x2.is_cuda and _tiles_fit(x2, w, bias)
 
 
 def _tiles(out, x2, w, bias, n, epilogue, what):
