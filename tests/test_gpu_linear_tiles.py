@@ -141,6 +141,24 @@ def test_wrong_bias_is_an_error(features):
         fused_ops.linear(x, w, mk(3, features))
 
 
+@pytest.mark.parametrize("rows", [40, 300])
+def test_rotary_tables_of_different_length(rows):
+    """An error for a prompt, as in rope(); few rows at positions inside both
+    tables are rotated."""
+    x, w = mk(1, rows, 128), mk(2, 96, 128, std=128 ** -0.5)
+    pos = torch.arange(rows, dtype=torch.int32, device=DEV) % 30
+    cos, sin = torch.rand(50, 16, device=DEV), torch.rand(30, 16, device=DEV)
+    with torch.no_grad():
+        if rows > 256:
+            with pytest.raises(ValueError, match="equal shape"):
+                fused_ops.linear_rope_qkv(x, w, None, pos, cos, sin, 1, 1, 32)
+            return
+        got = fused_ops.linear_rope_qkv(x, w, None, pos, cos, sin, 1, 1, 32)
+        want = fused_ops.linear_rope_qkv(x, w, None, pos, cos[:30].contiguous(), sin, 1, 1, 32)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 def test_refusals():
     L = _native.lib()
     x, w, out = mk(1, 64, 48), mk(2, 16, 48), torch.empty(64, 16, device=DEV)

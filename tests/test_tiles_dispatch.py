@@ -22,3 +22,15 @@ def test_other_biases_do_not_fit(shape):
     # one value per weight row is all the kernel reads
     x, w = operands()
     assert not fused_ops._tiles_fit(x, w, torch.randn(shape))
+
+
+def test_rotary_tables():
+    """A prompt's projection refuses tables of different length, as rope()
+    does; the few-row kernels rotate at the positions both tables hold."""
+    cos, sin = torch.randn(50, 16), torch.randn(40, 16)
+    with pytest.raises(ValueError, match="equal shape"):
+        fused_ops._rope_tables(cos, sin, 32, "rope", True)
+    assert fused_ops._rope_tables(cos, sin, 32, "rope", False)[2] == 40
+    assert fused_ops._rope_tables(cos, cos, 32, "rope", True)[2] == 50
+    with pytest.raises(ValueError, match="fp32"):
+        fused_ops._rope_tables(cos.double(), sin, 32, "rope", False)

@@ -137,6 +137,17 @@ def rope(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor, cos: torch.T
     return (q_out, k_out) if v is None else (q_out, k_out, v_out)
 
 
+def _rope_tables(cos, sin, d, what, equal):
+    """The fp32 tables as contiguous [max_pos, d/2] and the positions both hold.
+    equal: tables of different length are an error, as in rope()."""
+    if cos.dtype != torch.float32 or sin.dtype != torch.float32:
+        raise ValueError(f"{what}: cos / sin must be fp32 tables")
+    cos2, sin2 = cos.reshape(-1, d // 2).contiguous(), sin.reshape(-1, d // 2).contiguous()
+    if equal and cos2.shape != sin2.shape:
+        raise ValueError(f"{what}: cos / sin must be tables of equal shape [max_pos, D/2]")
+    return cos2, sin2, min(cos2.shape[0], sin2.shape[0])
+
+
 def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """gate * sigmoid(gate) * up in fp32, rounded once
     (kernels/fused_swiglu/kernel.py:6-19). gate and up may be strided column
@@ -290,9 +301,7 @@ def linear_rope_qkv(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: torch.Tensor | 
         return rope(qkv[:, :nq], qkv[:, nq:nq + nk], positions, cos, sin, v=qkv[:, nq + nk:],
                     hq=hq, hkv=hkv, d=d)
     _native.require_device(x2, w_qkv, positions, cos, sin, what="linear_rope_qkv")
-    if cos.dtype != torch.float32 or sin.dtype != torch.float32:
-        raise ValueError("linear_rope_qkv: cos / sin must be fp32 tables")
-    cos2, sin2 = cos.reshape(-1, d // 2).contiguous(), sin.reshape(-1, d // 2).contiguous()
+    cos2, sin2, max_pos = _rope_tables(cos, sin, d, "linear_rope_qkv", not few)
     pos = positions if positions.dtype == torch.int32 else positions.to(torch.int32)
     pos = pos.contiguous()
     if pos.numel() != T:
@@ -304,7 +313,7 @@ def linear_rope_qkv(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: torch.Tensor | 
     rc = fn(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), x2.data_ptr(), w_qkv.data_ptr(),
         _native.ptr(b_qkv), T, x2.shape[1], _x_stride(x2), pos.data_ptr(), cos2.data_ptr(),
-        sin2.data_ptr(), cos2.shape[0], hq, hkv, d, _native.dtype_code(x.dtype), None,
+        sin2.data_ptr(), max_pos, hq, hkv, d, _native.dtype_code(x.dtype), None,
         _native.stream_ptr(x.device))
     _native.check(rc, "linear_rope_qkv")
     return q, k, v
@@ -380,9 +389,7 @@ def linear_rope_qkv_rmsnorm(x: torch.Tensor, norm_weight: torch.Tensor, eps: flo
                                hq, hkv, d)
     _native.require_device(x2, norm_weight, w_qkv, positions, cos, sin,
                            what="linear_rope_qkv_rmsnorm")
-    if cos.dtype != torch.float32 or sin.dtype != torch.float32:
-        raise ValueError("linear_rope_qkv_rmsnorm: cos / sin must be fp32 tables")
-    cos2, sin2 = cos.reshape(-1, d // 2).contiguous(), sin.reshape(-1, d // 2).contiguous()
+    cos2, sin2, max_pos = _rope_tables(cos, sin, d, "linear_rope_qkv_rmsnorm", False)
     pos = positions if positions.dtype == torch.int32 else positions.to(torch.int32)
     pos = pos.contiguous()
     if pos.numel() != T:
@@ -393,7 +400,7 @@ def linear_rope_qkv_rmsnorm(x: torch.Tensor, norm_weight: torch.Tensor, eps: flo
     rc = _native.calls().pkv_linear_rope_qkv_rmsnorm(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), x2.data_ptr(), norm_weight.data_ptr(),
         float(eps), w_qkv.data_ptr(), _native.ptr(b_qkv), T, x2.shape[1], _x_stride(x2),
-        pos.data_ptr(), cos2.data_ptr(), sin2.data_ptr(), cos2.shape[0], hq, hkv, d,
+        pos.data_ptr(), cos2.data_ptr(), sin2.data_ptr(), max_pos, hq, hkv, d,
         _native.dtype_code(x.dtype), None, _native.stream_ptr(x.device))
     _native.check(rc, "linear_rope_qkv_rmsnorm")
     return q, k, v
