@@ -141,6 +141,14 @@ def test_wrong_bias_is_an_error(features):
         fused_ops.linear(x, w, mk(3, features))
 
 
+def test_trace_records_the_product():
+    """A traced projection answers for other inputs than the traced one."""
+    x, x1, w = mk(1, 300, 128), mk(3, 300, 128), mk(2, 96, 128, std=128 ** -0.5)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda a: fused_ops.linear(a, w), x, check_trace=False)
+        torch.testing.assert_close(traced(x1).double(), x1.double() @ w.double().t(), **TOL)
+
+
 @pytest.mark.parametrize("rows", [40, 300])
 def test_rotary_tables_of_different_length(rows):
     """An error for a prompt, as in rope(); few rows at positions inside both

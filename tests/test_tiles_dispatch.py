@@ -3,6 +3,10 @@ CPU: what it refuses goes to the framework's linear, which answers or raises
 as it does by itself."""
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
+from torch.utils.flop_counter import FlopCounterMode
 
 from serving import fused_ops
 
@@ -34,3 +38,55 @@ def test_rotary_tables():
     assert fused_ops._rope_tables(cos, cos, 32, "rope", True)[2] == 50
     with pytest.raises(ValueError, match="fp32"):
         fused_ops._rope_tables(cos.double(), sin, 32, "rope", False)
+
+
+class Dispatch(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class Function(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("mode", [Dispatch, Function, lambda: FlopCounterMode(display=False)])
+def test_modes_see_the_framework(mode):
+    x, w = operands()
+    with mode():
+        assert not fused_ops._tiles_fit(x, w, None)
+    assert fused_ops._tiles_fit(x, w, None)
+
+
+def test_default_device_is_no_transform():
+    x, w = operands()
+    with torch.device("cpu"):
+        assert fused_ops._tiles_fit(x, w, None)
+
+
+@pytest.mark.parametrize("trace", [
+    lambda f, x: torch.jit.trace(f, x, check_trace=False),
+    lambda f, x: make_fx(f)(x),
+    lambda f, x: make_fx(f, pre_dispatch=True)(x),
+    lambda f, x: torch.compile(f, backend="eager", fullgraph=True)(x),
+    lambda f, x: torch.export.export(Module(f), (x,))])
+def test_traces_hold_the_framework_call(trace):
+    """A trace would hold an empty tensor in the place of a kernel's output."""
+    x, w = operands()
+    seen = []
+
+    def f(a):
+        fits = fused_ops._tiles_fit(a, w, None)
+        seen.append(fits)
+        return torch.nn.functional.linear(a, w)
+    trace(f, x)
+    assert seen and not any(seen)
+
+
+class Module(torch.nn.Module):
+    def __init__(self, f):
+        super().__init__()
+        self.f = f
+
+    def forward(self, x):
+        return self.f(x)

@@ -17,6 +17,7 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _native
 
@@ -199,10 +200,23 @@ TILES_SMALL_K = 512
 TILES_MIN_ROWS = 1024
 
 
+def _mode_active() -> bool:
+    """Whether a dispatch or function mode is to see the framework's calls. The
+    one behind torch.set_default_device only places new tensors."""
+    if (torch._C._len_torch_dispatch_stack() != 0
+            or torch._ops._len_torch_dispatch_stack_pre_dispatch() != 0):
+        return True
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+               for i in range(torch._C._len_torch_function_stack()))
+
+
 def _transformed(ts) -> bool:
-    """Whether a call records, transforms or casts these tensors: gradients,
-    torch.func and forward-mode AD, autocast, tensor subclasses (tracing)."""
-    return ((torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+    """Whether a call records, transforms or casts these tensors: compilation
+    and tracing (where the tensors can be plain ones: torch.jit.trace, make_fx),
+    modes, gradients, torch.func and forward-mode AD, autocast, tensor
+    subclasses. A kernel call would be missing from what they record."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or _mode_active()
+            or (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
             or torch.is_autocast_enabled() or forward_ad._current_level >= 0
             or torch._C._functorch.peek_interpreter_stack() is not None
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in ts))
