@@ -141,6 +141,25 @@ def test_wrong_bias_is_an_error(features):
         fused_ops.linear(x, w, mk(3, features))
 
 
+def test_residual_update_is_seen_by_autograd():
+    """A backward whose graph saved the residual raises, as after add_; an
+    inference tensor outside inference mode is refused."""
+    x, w, r = mk(1, 300, 128), mk(2, 96, 128, std=128 ** -0.5), mk(3, 300, 96)
+    p = torch.ones(300, 96, device=DEV, requires_grad=True)
+    y = (p * r).sum()  # saves r
+    with torch.no_grad():
+        before = r._version
+        fused_ops.linear_residual_(r, x, w)
+    assert r._version == before + 1
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        y.backward()
+    with torch.inference_mode():
+        q = torch.zeros(300, 96, device=DEV)
+        fused_ops.linear_residual_(q, x, w)
+    with torch.no_grad(), pytest.raises(RuntimeError, match="inference"):
+        fused_ops.linear_residual_(q, x, w)
+
+
 def test_trace_records_the_product():
     """A traced projection answers for other inputs than the traced one."""
     x, x1, w = mk(1, 300, 128), mk(3, 300, 128), mk(2, 96, 128, std=128 ** -0.5)

@@ -90,3 +90,12 @@ class Module(torch.nn.Module):
 
     def forward(self, x):
         return self.f(x)
+
+
+def test_inference_residual_is_the_frameworks():
+    x, _ = operands()
+    with torch.inference_mode():
+        r = torch.zeros(300, 96)
+        assert fused_ops._tiles_resid_fit(r, x, 96)
+    assert not fused_ops._tiles_resid_fit(r, x, 96)
+    assert fused_ops._tiles_resid_fit(torch.zeros(300, 96), x, 96)

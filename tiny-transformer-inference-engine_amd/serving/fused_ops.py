@@ -344,6 +344,18 @@ def _norm_ok(x2: torch.Tensor, norm_weight: torch.Tensor) -> bool:
             and norm_weight.data_ptr() % 16 == 0)
 
 
+def _tiles_resid_fit(resid: torch.Tensor, x2: torch.Tensor, n: int) -> bool:
+    """Whether the tile kernel may update resid in place where add_ did: an
+    inference tensor outside inference mode is add_'s error."""
+    return (resid.is_contiguous() and resid.dtype == x2.dtype and resid.device == x2.device
+            and resid.numel() == x2.shape[0] * n
+            and (not resid.is_inference() or torch.is_inference_mode_enabled())
+            and not _transformed((resid,))
+            # in place, and other workgroups still read x
+            and resid.untyped_storage().data_ptr() != x2.untyped_storage().data_ptr()
+            and resid.data_ptr() % 16 == 0)
+
+
 def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
                      bias: torch.Tensor | None = None) -> torch.Tensor:
     """resid += x W^T + b in place, the projection rounded to resid.dtype
@@ -354,14 +366,11 @@ def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
     n = weight.shape[0]
     if (not _linear_ok(x2, weight, bias, n) or not resid.is_contiguous()
             or resid.dtype != x.dtype or resid.numel() != x2.shape[0] * n):
-        if (resid.is_contiguous() and resid.dtype == x.dtype and resid.device == x.device
-                and resid.numel() == x2.shape[0] * n and resid.data_ptr() % 16 == 0
-                and not _transformed((resid,))
-                # in place, and other workgroups still read x
-                and resid.untyped_storage().data_ptr() != x2.untyped_storage().data_ptr()
-                and _tiles_ok(x2, weight, bias)):
-            return _tiles(resid, x2, weight, bias, n, _native.EPILOGUE_RESIDUAL,
-                          "linear_residual_")
+        if _tiles_resid_fit(resid, x2, n) and _tiles_ok(x2, weight, bias):
+            _tiles(resid, x2, weight, bias, n, _native.EPILOGUE_RESIDUAL, "linear_residual_")
+            # as add_ does: a graph that saved resid finds it changed
+            torch.autograd.graph.increment_version(resid)
+            return resid
         return resid.add_(linear(x, weight, bias).view(resid.shape))
     rc = _native.calls().pkv_linear_residual(
         resid.data_ptr(), x2.data_ptr(), weight.data_ptr(), _native.ptr(bias), x2.shape[0], n,
