@@ -12,6 +12,8 @@ from serving import _native, fused_ops
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 TOL = dict(rtol=2e-5, atol=2e-5)
+# weights of variance 1 in the place of 1/128: sqrt(128) times the sums
+WIDE = {False: TOL, True: dict(rtol=2.4e-4, atol=2.4e-4)}
 
 
 def mk(seed, *shape, std=1.0):
@@ -158,6 +160,26 @@ def test_residual_update_is_seen_by_autograd():
         fused_ops.linear_residual_(q, x, w)
     with torch.no_grad(), pytest.raises(RuntimeError, match="inference"):
         fused_ops.linear_residual_(q, x, w)
+
+
+@pytest.mark.parametrize("shared", ["x", "weight", "bias", "rows of x"])
+def test_residual_sharing_memory_is_read_first(shared):
+    """resid may be an operand itself: every operand is read before it changes."""
+    x, w, b = mk(1, 1024, 128), mk(2, 128, 128, std=128 ** -0.5), mk(3, 128)
+    r = mk(4, 1024, 128)
+    if shared == "x":
+        r = x
+    elif shared == "weight":
+        w = r[300:428]
+    elif shared == "bias":
+        b = r[700]
+    else:
+        buf = mk(5, 2048, 128)
+        x, r = buf[:1024], buf[1023:2047]
+    want = r.double() + x.double() @ w.double().t() + b.double()
+    with torch.no_grad():
+        got = fused_ops.linear_residual_(r, x, w, b)
+    torch.testing.assert_close(got.double(), want, **WIDE[shared == "weight"])
 
 
 def test_trace_records_the_product():

@@ -99,3 +99,16 @@ def test_inference_residual_is_the_frameworks():
         assert fused_ops._tiles_resid_fit(r, x, 96)
     assert not fused_ops._tiles_resid_fit(r, x, 96)
     assert fused_ops._tiles_resid_fit(torch.zeros(300, 96), x, 96)
+
+
+def test_memory_apart():
+    buf = torch.zeros(1000)
+    out = buf[100:200]
+    assert fused_ops._apart(out, None)
+    assert fused_ops._apart(out, buf[:100]) and fused_ops._apart(out, buf[200:])
+    assert not fused_ops._apart(out, buf[:101]) and not fused_ops._apart(out, buf[199:])
+    assert not fused_ops._apart(out, out)
+    # rows of 10 every 60 elements, the last ones past out's start
+    assert fused_ops._apart(out, buf.as_strided((2, 10), (60, 1)))
+    assert not fused_ops._apart(out, buf.as_strided((3, 10), (60, 1)))
+    assert fused_ops._apart(out, buf[150:150])

@@ -351,9 +351,18 @@ def _tiles_resid_fit(resid: torch.Tensor, x2: torch.Tensor, n: int) -> bool:
             and resid.numel() == x2.shape[0] * n
             and (not resid.is_inference() or torch.is_inference_mode_enabled())
             and not _transformed((resid,))
-            # in place, and other workgroups still read x
-            and resid.untyped_storage().data_ptr() != x2.untyped_storage().data_ptr()
             and resid.data_ptr() % 16 == 0)
+
+
+def _apart(out: torch.Tensor, t) -> bool:
+    """Whether the memory of t (None, or a tensor without negative strides) lies
+    outside the contiguous out's: workgroups write out while others read t."""
+    if t is None or t.numel() == 0:
+        return True
+    last = sum((n - 1) * s for n, s in zip(t.shape, t.stride()))
+    a, b = out.data_ptr(), t.data_ptr()
+    return (b + (last + 1) * t.element_size() <= a
+            or a + out.numel() * out.element_size() <= b)
 
 
 def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
@@ -366,7 +375,8 @@ def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
     n = weight.shape[0]
     if (not _linear_ok(x2, weight, bias, n) or not resid.is_contiguous()
             or resid.dtype != x.dtype or resid.numel() != x2.shape[0] * n):
-        if _tiles_resid_fit(resid, x2, n) and _tiles_ok(x2, weight, bias):
+        if (_tiles_resid_fit(resid, x2, n) and _tiles_ok(x2, weight, bias)
+                and _apart(resid, x2) and _apart(resid, weight) and _apart(resid, bias)):
             _tiles(resid, x2, weight, bias, n, _native.EPILOGUE_RESIDUAL, "linear_residual_")
             # as add_ does: a graph that saved resid finds it changed
             torch.autograd.graph.increment_version(resid)
