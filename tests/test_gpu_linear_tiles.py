@@ -182,6 +182,18 @@ def test_residual_sharing_memory_is_read_first(shared):
     torch.testing.assert_close(got.double(), want, **WIDE[shared == "weight"])
 
 
+def test_forms_of_the_framework():
+    """A vector as the weight, no features, empty sums, negated views."""
+    x, w, b = mk(1, 300, 128), mk(2, 96, 128, std=128 ** -0.5), mk(3, 96)
+    with torch.no_grad():
+        torch.testing.assert_close(fused_ops.linear(x, w[0]).double(), x.double() @ w[0].double(),
+                                   **TOL)
+        assert fused_ops.linear(x, w[:0]).shape == (300, 0)
+        assert torch.equal(fused_ops.linear(x[:, :0], w[:, :0], b), b.expand(300, 96))
+        got = fused_ops.linear(torch._neg_view(x), w)
+        torch.testing.assert_close(got.double(), -(x.double() @ w.double().t()), **TOL)
+
+
 def test_trace_records_the_product():
     """A traced projection answers for other inputs than the traced one."""
     x, x1, w = mk(1, 300, 128), mk(3, 300, 128), mk(2, 96, 128, std=128 ** -0.5)

@@ -28,6 +28,20 @@ def test_other_biases_do_not_fit(shape):
     assert not fused_ops._tiles_fit(x, w, torch.randn(shape))
 
 
+def test_forms_only_the_framework_takes():
+    x, w = operands()
+    assert not fused_ops._tiles_fit(x, w[0], None)                    # a vector
+    assert not fused_ops._tiles_fit(x, w[:0], None)                   # no features
+    assert not fused_ops._tiles_fit(x[:, :0], w[:, :0], None)         # empty sums
+    assert not fused_ops._tiles_fit(x, w.to_sparse(), None)
+    assert not fused_ops._tiles_fit(x, w[:, :96], None)               # an error there
+    assert not fused_ops._tiles_fit(torch._neg_view(x), w, None)
+    assert not fused_ops._tiles_fit(x, torch._neg_view(w), None)
+    assert not fused_ops._tiles_resid_fit(torch._neg_view(torch.zeros(300, 96)), x, 96)
+    assert not fused_ops._tiles_fit(x.double(), w.double(), None)
+    assert not fused_ops._tiles_fit(x[:256], w, None)
+
+
 def test_rotary_tables():
     """A prompt's projection refuses tables of different length, as rope()
     does; the few-row kernels rotate at the positions both tables hold."""

@@ -223,19 +223,20 @@ def _transformed(ts) -> bool:
 
 
 def _tiles_fit(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
-    """Whether pkv_linear_tiles takes a projection of these operands; calls the
-    framework has to see stay on its GEMM, and so does a bias of any other shape
-    than one value per weight row, which is all the kernel reads."""
+    """Whether pkv_linear_tiles takes a projection of these operands. Calls the
+    framework has to see stay on its GEMM, and so do forms that only it takes: a
+    bias of any other shape than one value per weight row (all the kernel reads),
+    a weight that is a vector, sparse or empty, and lazily negated values."""
     ts = (x2, w) if bias is None else (x2, w, bias)
     rows, k = x2.shape
     return (rows > (LINEAR_MAX_ROWS if k <= TILES_SMALL_K else TILES_MIN_ROWS)
-            and k <= TILES_MAX_K
-            and all(t.dtype == torch.float32 and t.device == x2.device for t in ts)
-            and not _transformed(ts)
+            and 0 < k <= TILES_MAX_K
+            and all(t.dtype == torch.float32 and t.device == x2.device
+                    and t.layout is torch.strided for t in ts)
+            and not _transformed(ts) and not any(t.is_neg() for t in ts)
+            and w.dim() == 2 and w.shape[1] == k and k % 32 == 0
+            and 0 < w.shape[0] <= LINEAR_MAX_FEATURES and w.is_contiguous()
             and (bias is None or (bias.shape == w.shape[:1] and bias.is_contiguous()))
-            and w.is_contiguous()
-            and w.shape[1] == k and k % 32 == 0
-            and w.shape[0] <= LINEAR_MAX_FEATURES
             and x2.stride(0) >= k and x2.stride(0) % 4 == 0
             and rows * x2.stride(0) < 1 << 29 and w.numel() < 1 << 29
             and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
@@ -350,7 +351,7 @@ def _tiles_resid_fit(resid: torch.Tensor, x2: torch.Tensor, n: int) -> bool:
     return (resid.is_contiguous() and resid.dtype == x2.dtype and resid.device == x2.device
             and resid.numel() == x2.shape[0] * n
             and (not resid.is_inference() or torch.is_inference_mode_enabled())
-            and not _transformed((resid,))
+            and not _transformed((resid,)) and not resid.is_neg()
             and resid.data_ptr() % 16 == 0)
 
 
