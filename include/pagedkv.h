@@ -190,7 +190,9 @@ int pkv_gather(void* k_out, void* v_out, const void* k_pool,
 
 /*
  * Bytes of workspace pkv_paged_attention needs for this problem (0 when no
- * sequence is split). `max_kv_len` <= 0 means max_blk * block_size.
+ * sequence is split), whatever the alignment of its tensors: head dims 32, 64
+ * and 128 with tensors that are not 16-byte aligned split contexts finer, and
+ * in the aligned tensors' coarser pieces where the workspace is smaller. `max_kv_len` <= 0 means max_blk * block_size.
  * The workspace holds partial results and, in its first 256 KiB, the
  * persistent kernel's per-sequence arrival counters: zero-fill it once
  * before its first use; every call leaves the counters zero again. Calls
@@ -279,7 +281,8 @@ int pkv_paged_attention_append(void* out, float* lse, const void* q,
  * status bits as pkv_paged_attention; its split-K partials and arrival
  * counters live in a 16 MiB scratch array the library holds on every device
  * it runs on, for the life of the process. A problem whose
- * pkv_attention_workspace_bytes() exceeds 16 MiB returns PKV_ERR_WORKSPACE.
+ * partials (in the coarser pieces, see pkv_attention_workspace_bytes()) exceed
+ * 16 MiB returns PKV_ERR_WORKSPACE.
  * The call allocates nothing. The array starts zero-filled (static storage
  * of the library's code object) and every call leaves its counter header at
  * zero; the first call on a device takes the array's address and zeroes that

@@ -70,6 +70,13 @@ def test_validation_errors_without_gpu():
     assert L.pkv_append(None, None, 10, None, None, None, 0, 64, 2, None, None) == 0
 
 
+def test_workspace_holds_the_row_kernels_partitions():
+    """Tensors that are not 16-byte aligned take the row kernel, which splits a
+    prompt of 500 tokens (125 tiles of 8 heads) into 64-token partitions."""
+    ws = _native.lib().pkv_attention_workspace_bytes(1, 500, 8, 1, 64, 32, 16, 500, 0, 0)
+    assert ws >= 125 * 8 * 32 * (64 + 2) * 4
+
+
 def test_workspace_sizing():
     L = _native.lib()
     # a single partition needs no workspace

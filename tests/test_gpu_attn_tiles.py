@@ -169,3 +169,30 @@ def test_unaligned_tensors_take_the_row_kernel():
     assert q.data_ptr() % 16 != 0
     p["q"] = q
     check(p, torch.float32)
+
+
+@pytest.mark.parametrize("q_lens,pasts", [([500], [0]), ([8, 8], [2000, 1500]), ([1, 40], [900, 3])])
+@pytest.mark.parametrize("workspace", [True, False])
+def test_unaligned_tensors_split(q_lens, pasts, workspace):
+    # the row kernel in its own partitions, and unsplit where no workspace is given
+    p = problem(q_lens, pasts, 8, 1, 64, 16, torch.float32)
+    q = torch.empty(p["q"].numel() + 1, device=DEV)[1:].view(p["q"].shape)
+    q.copy_(p["q"])
+    out = torch.empty_like(p["q"])
+    L, n, mk = _native.lib(), len(q_lens), max(a + b for a, b in zip(q_lens, pasts))
+    if not workspace:
+        mk = min(mk, 512)  # the tile rule's one piece; longer contexts grow it
+    wsb = L.pkv_attention_workspace_bytes(n, p["max_q"], 8, 1, 64, p["table"].shape[1], 16, mk, 0,
+                                          0)
+    ws = torch.zeros(wsb, dtype=torch.uint8, device=DEV) if workspace else None
+    assert wsb > 0
+    rc = L.pkv_paged_attention(
+        out.data_ptr(), None, q.data_ptr(), p["k"].data_ptr(), p["v"].data_ptr(),
+        p["k"].shape[0], 16, p["table"].data_ptr(), p["table"].shape[1], p["lens"].data_ptr(),
+        p["qsl"].data_ptr(), n, q.shape[0], p["max_q"], mk, 8, 1, 64, 0.0, 1, 0, 0,
+        _native.ptr(ws), wsb if workspace else 0, None, _native.stream_ptr(q.device))
+    _native.check(rc, "pkv_paged_attention")
+    want, _ = ref.paged_attention(np64(p["q"]), np64(p["k"]), np64(p["v"]),
+                                  p["table"].cpu().numpy(), p["lens"].cpu().numpy(),
+                                  p["qsl"].cpu().numpy())
+    np.testing.assert_allclose(np64(out), want, rtol=1e-5, atol=1e-5)

@@ -328,7 +328,7 @@ bool sk_fits(int64_t virt, int max_blk) {
 
 AttnPlan plan_attention(int n_seq, int max_q_len, int hq, int hkv, int d,
                         int max_blk, int block_size, int max_kv_len,
-                        int part_tokens, int dtype) {
+                        int part_tokens, int dtype, bool aligned) {
   AttnPlan p{};
   // fp8 pools are read by the MFMA kernels only (rows widened in LDS)
   const bool kv8 = dtype_kv8(dtype);
@@ -415,13 +415,15 @@ AttnPlan plan_attention(int n_seq, int max_q_len, int hq, int hkv, int d,
     plen = 512;
     while (plen < 4096 && (int64_t)plen * 8 < kvb) plen *= 2;
   } else if (plen <= 0) {
-    // The tile kernel (head dim 32 / 64 / 128) splits a context only where
-    // its tiles leave CUs idle, into pieces of at least 512 tokens: its four
-    // wavefronts already share them, and the merge launch costs ~5 us (one
-    // prompt of 500 tokens 20 us split in two, 15 whole). The row kernel aims
-    // for ~2048 workgroups, so the 256 CUs stay busy even when most sequences
-    // are far below the bound.
-    const bool tiles = d == 32 || d == 64 || d == 128;
+    // The tile kernel (head dim 32 / 64 / 128, aligned tensors) splits a
+    // context only where its tiles leave CUs idle, into pieces of at least 512
+    // tokens: its four wavefronts already share them, and the merge launch
+    // costs ~5 us (one prompt of 500 tokens 20 us split in two, 15 whole). The
+    // row kernel aims for ~2048 workgroups, so the 256 CUs stay busy even when
+    // most sequences are far below the bound (in the tile kernel's pieces it
+    // takes 137 us for one unaligned fp32 prompt of 500 tokens, 8 heads of 64,
+    // in its own 45; 2 x 8 rows behind 2000 tokens 141 and 30).
+    const bool tiles = aligned && (d == 32 || d == 64 || d == 128);
     int64_t parts_target = ((tiles ? 256 : 2048) + units - 1) / (units > 0 ? units : 1);
     if (parts_target < 1) parts_target = 1;
     plen = (int)((kvb + parts_target - 1) / parts_target);
@@ -441,20 +443,20 @@ AttnPlan plan_attention(int n_seq, int max_q_len, int hq, int hkv, int d,
 
 AttnSplit plan_split(int n_seq, int max_q_len, int hq, int hkv, int d, int max_blk,
                      int block_size, int max_kv_len, int part_tokens, int dtype,
-                     bool has_qloc) {
+                     bool has_qloc, bool aligned) {
   AttnSplit sp{};
   sp.mixed = has_qloc && max_q_len > 1 && n_seq >= 2 && max_blk >= 1 &&
              decode_mfma_supported(dtype_base(dtype), 1, hq / hkv, d);
   if (!sp.mixed) {
     sp.dec = plan_attention(n_seq, max_q_len, hq, hkv, d, max_blk, block_size, max_kv_len,
-                            part_tokens, dtype);
+                            part_tokens, dtype, aligned);
     sp.ws_bytes = sp.dec.ws_bytes;
     return sp;
   }
   sp.dec = plan_attention(n_seq, 1, hq, hkv, d, max_blk, block_size, max_kv_len, part_tokens,
-                          dtype);
+                          dtype, aligned);
   sp.pre = plan_attention(n_seq, max_q_len, hq, hkv, d, max_blk, block_size, max_kv_len,
-                          part_tokens, dtype);
+                          part_tokens, dtype, aligned);
   sp.ws_bytes = sp.dec.ws_bytes > sp.pre.ws_bytes ? sp.dec.ws_bytes : sp.pre.ws_bytes;
   return sp;
 }

@@ -611,13 +611,17 @@ int launch_t(const AttnArgs& a, const AttnPlan& p, hipStream_t stream) {
 
 }  // namespace
 
+bool attn_tiles_aligned(const void* q, const void* out, const void* k_pool, const void* v_pool) {
+  // every row is a multiple of 64 bytes
+  return ((uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pool | (uintptr_t)v_pool) % 16 == 0;
+}
+
 bool attn_tiles_supported(const AttnArgs& a, int dtype) {
   // the row kernel takes what is left: other head dims, and a pool, q or out
-  // that is not 16-byte aligned (every row is a multiple of 64 bytes)
-  const uintptr_t p = (uintptr_t)a.q | (uintptr_t)a.out | (uintptr_t)a.k_pool |
-                      (uintptr_t)a.v_pool;
+  // that is not 16-byte aligned
   return (dtype == PKV_DTYPE_F32 || dtype == PKV_DTYPE_BF16 || dtype == PKV_DTYPE_F16) &&
-         !a.kv8 && (a.d == 32 || a.d == 64 || a.d == 128) && p % 16 == 0;
+         !a.kv8 && (a.d == 32 || a.d == 64 || a.d == 128) &&
+         attn_tiles_aligned(a.q, a.out, a.k_pool, a.v_pool);
 }
 
 int launch_attn_tiles(const AttnArgs& a, const AttnPlan& p, int dtype, hipStream_t stream) {

@@ -138,9 +138,10 @@ size_t pkv_attention_workspace_bytes(int n_seq, int max_q_len, int hq, int hkv,
   if (n_seq <= 0 || max_q_len <= 0 || hkv <= 0 || hq <= 0 || hq % hkv != 0 ||
       part_tokens < PKV_PART_STREAM)
     return 0;
-  // query_start_loc is required whenever max_q_len > 1
+  // query_start_loc is required whenever max_q_len > 1; enough for tensors of
+  // any alignment
   return plan_split(n_seq, max_q_len, hq, hkv, d, max_blk, block_size, max_kv_len,
-                    part_tokens, dtype, max_q_len > 1)
+                    part_tokens, dtype, max_q_len > 1, false)
       .ws_bytes;
 }
 
@@ -185,8 +186,14 @@ int attention_impl(void* out, float* lse, const void* q, const void* k_pool,
     return fail(PKV_ERR_INVALID, "null pointer argument");
   if (!query_start_loc && max_q_len != 1)
     return fail(PKV_ERR_INVALID, "query_start_loc may be NULL only when max_q_len == 1");
-  const AttnSplit sp = plan_split(n_seq, max_q_len, hq, hkv, d, max_blk, block_size,
-                                  max_kv_len, part_tokens, dtype, query_start_loc != nullptr);
+  // unaligned tensors take the row kernel, in the tile kernel's coarser
+  // partitions where the workspace does not hold its own
+  const bool aligned = attn_tiles_aligned(q, out, k_pool, v_pool);
+  AttnSplit sp = plan_split(n_seq, max_q_len, hq, hkv, d, max_blk, block_size, max_kv_len,
+                            part_tokens, dtype, query_start_loc != nullptr, aligned);
+  if (!aligned && sp.ws_bytes > (workspace ? workspace_bytes : 0))
+    sp = plan_split(n_seq, max_q_len, hq, hkv, d, max_blk, block_size, max_kv_len, part_tokens,
+                    dtype, query_start_loc != nullptr, true);
   if (sp.ws_bytes > 0 && (!workspace || workspace_bytes < sp.ws_bytes))
     return fail(PKV_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given",
                 sp.ws_bytes, workspace ? workspace_bytes : (size_t)0);
@@ -366,7 +373,8 @@ int pkv_paged_attention_noalloc(void* out, float* lse, const void* q, const void
   if (n_seq > 0 && max_q_len > 0 && hkv > 0 && hq > 0 && hq % hkv == 0 &&
       part_tokens >= PKV_PART_STREAM) {
     const size_t need = plan_split(n_seq, max_q_len, hq, hkv, d, max_blk, block_size,
-                                   max_kv_len, part_tokens, dtype, query_start_loc != nullptr)
+                                   max_kv_len, part_tokens, dtype, query_start_loc != nullptr,
+                                   true)
                             .ws_bytes;
     if (need > kScratchBytes)
       return fail(PKV_ERR_WORKSPACE,

@@ -330,11 +330,14 @@ int launch_decode_small(const AttnArgs& a, const AttnPlan& p, int dtype, hipStre
 // matrix cores, any group size, head dim 32 / 64 / 128; needs 16-byte aligned
 // pools, q and out.
 bool attn_tiles_supported(const AttnArgs& a, int dtype);
+bool attn_tiles_aligned(const void* q, const void* out, const void* k_pool, const void* v_pool);
 int launch_attn_tiles(const AttnArgs& a, const AttnPlan& p, int dtype, hipStream_t stream);
 
+// aligned: attn_tiles_aligned's tensors. Without it the row kernel runs, whose
+// partitions are finer: the larger need of workspace.
 AttnPlan plan_attention(int n_seq, int max_q_len, int hq, int hkv, int d,
                         int max_blk, int block_size, int max_kv_len,
-                        int part_tokens, int dtype);
+                        int part_tokens, int dtype, bool aligned);
 
 // A batch that may mix single-token (decode) and multi-token (prefill)
 // queries is split when the decode sequences can take an MFMA decode
@@ -349,7 +352,7 @@ struct AttnSplit {
 };
 AttnSplit plan_split(int n_seq, int max_q_len, int hq, int hkv, int d, int max_blk,
                      int block_size, int max_kv_len, int part_tokens, int dtype,
-                     bool has_qloc);
+                     bool has_qloc, bool aligned);
 
 int launch_attention(const AttnArgs& a, const AttnPlan& plan, int dtype,
                      hipStream_t stream);
