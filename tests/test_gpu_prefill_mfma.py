@@ -86,3 +86,22 @@ def test_prefill_noncausal_and_scale(causal, scale):
                                  causal=causal)
     assert np.abs(np64(O) - eo).max() <= 2e-2
     np.testing.assert_allclose(L.cpu().numpy(), el, rtol=0, atol=2e-2)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("hq,dtype", [(16, torch.bfloat16), (32, torch.float16)])
+def test_short_tables_mask_alike(hq, dtype, causal):
+    """Tables of up to 128 tokens mask every chunk, longer ones the chunks a
+    range ends in: the same bits, and the oracle's values."""
+    p, q, qsl, mql = problem([(128, 128), (77, 77), (5, 40), (33, 97), (9, 9)], hq, 1, 128, 16,
+                             dtype, seed=43)
+    assert p.block_tables.shape[1] == 8
+    wide = torch.nn.functional.pad(p.block_tables, (0, 1)).contiguous()
+    O, L = paged_attn_fwd(q, p.k_pool, p.v_pool, p.block_tables, p.seq_lens, qsl, mql,
+                          causal=causal)
+    O1, L1 = paged_attn_fwd(q, p.k_pool, p.v_pool, wide, p.seq_lens, qsl, mql, causal=causal)
+    assert torch.equal(O, O1) and torch.equal(L, L1)
+    eo, _ = ref.paged_attention(np64(q), np64(p.k_pool), np64(p.v_pool),
+                                p.block_tables.cpu().numpy(), p.seq_lens.cpu().numpy(),
+                                qsl.cpu().numpy(), causal=causal)
+    assert np.abs(np64(O) - eo).max() <= 2e-2

@@ -156,17 +156,20 @@ __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_ex
 // Rows are padded by 16 bytes (PITCH = 2D + 16): row r starts 4r (mod 64)
 // banks further on for D = 128 (36r for D = 64), so the 16 rows an MFMA
 // fragment read touches at one 16-byte piece land on distinct bank groups.
-// V's rows are read by transposing reads, 32 bytes of each of 8 rows at once:
-// at D = 128 they are padded by 32 bytes, which puts the 8 on distinct banks
-// (by 16 bytes every bank was hit twice: 24 of 56 M LDS cycles of a long
-// prefill were conflicts); at D = 64 the 16 bytes already spread them. Every
-// fragment address is one base register plus an immediate offset.
-template <int D>
+// V's rows are read by transposing reads, 32 bytes of each of 8 rows at once.
+// PREFILL: at D = 128 they are padded by 32 bytes, which puts the 8 on
+// distinct banks (with 16 every bank is hit twice; at D = 64 the 16 already
+// spread them): 4 prompts of 1-4 K tokens x 32 heads of 128 take 484 us so, 510
+// with 16 bytes and the score mask on every chunk. Decode keeps 16: its few
+// chunks per wavefront wait for memory, and the wider rows cost a step of 8
+// sequences of 130 tokens x 32 heads 7.1 -> 7.2 us. Every fragment address is
+// one base register plus an immediate offset.
+template <int D, bool PREFILL = false>
 struct ChunkGeo {
   static constexpr int CPR = D / 8;                 // 16-byte pieces per row
   static constexpr int ROW_BYTES = D * 2;
-  static constexpr int PITCH = ROW_BYTES + 16;                      // K rows
-  static constexpr int VPITCH = ROW_BYTES + (D == 128 ? 32 : 16);  // V rows
+  static constexpr int PITCH = ROW_BYTES + 16;                                // K rows
+  static constexpr int VPITCH = ROW_BYTES + (PREFILL && D == 128 ? 32 : 16);  // V rows
   static constexpr int ROWS_PER_LOAD = 64 / CPR;    // rows one wave load covers
   static constexpr int NPL = kChunk / ROWS_PER_LOAD;  // loads per lane per tensor
   static constexpr int KBYTES = kChunk * PITCH;
@@ -436,13 +439,15 @@ __device__ __forceinline__ void chunk_scores(const ChunkCtx& cx,
 // Softmax update and O^T += V^T P^T for the chunk whose scores are sacc
 // (row tiles N0 ... N0 + NC - 1 of st): tokens seg_lo + 32c ..., those at or
 // past seg_hi[nt] masked out for row tile N0 + nt (each V^T fragment is
-// read once for all of them).
-template <typename T, int D, int NT, int N0, int NC, bool MASK>
+// read once for all of them). PREFILL: cx.vl has the prefill kernel's rows.
+// MASK: none, every chunk (without a branch), or the chunks a range ends in.
+enum { kMaskNone = 0, kMaskAll = 1, kMaskEnd = 2 };
+template <typename T, int D, int NT, int N0, int NC, int MASK, bool PREFILL = false>
 __device__ __forceinline__ void chunk_update_sub(int c, const ChunkCtx& cx,
                                                  const int (&seg_hi)[NC],
                                                  const floatx4 (&sacc)[NC][2],
                                                  WaveState<NT, D / 16>& st) {
-  using Geo = ChunkGeo<D>;
+  using Geo = ChunkGeo<D, PREFILL>;
   using v8 = typename Ops<T>::v8;
   constexpr int DT = D / 16;
 
@@ -465,10 +470,9 @@ __device__ __forceinline__ void chunk_update_sub(int c, const ChunkCtx& cx,
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) sv[nt][4 * h + rr] = sacc[nt][h][rr];
-    // uniform: the range ends inside the chunk (a mask on every chunk and the
-    // narrower V rows took 510 us on 4 prompts of 1-4 K tokens x 32 heads of
-    // 128; 484 without both)
-    if (MASK && cb + kChunk > seg_hi[nt]) {
+    // kMaskEnd's condition is the same in every lane (a row tile is one token's
+    // heads), and nothing under it needs that
+    if (MASK == kMaskAll || (MASK == kMaskEnd && cb + kChunk > seg_hi[nt])) {
       // token 16h + 4 grp + rr of the chunk is in range iff 16h + rr < lim
       const int lim = seg_hi[nt] - cb - 4 * cx.grp;
 #pragma unroll
@@ -540,7 +544,9 @@ __device__ __forceinline__ void chunk_update(int c, const ChunkCtx& cx,
   int seg_hi[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) seg_hi[nt] = cx.seg_hi;
-  chunk_update_sub<T, D, NT, 0, NT, MASK>(c, cx, seg_hi, sacc, st);
+  // without a branch: the masked chunks are the last of a range, short contexts
+  // have no others (a branch cost steps of up to 700 tokens at D = 128 1-2%)
+  chunk_update_sub<T, D, NT, 0, NT, MASK ? kMaskAll : kMaskNone>(c, cx, seg_hi, sacc, st);
 }
 
 // QK / softmax / PV of the chunk staged in cx's slices.

@@ -60,7 +60,7 @@ inline int64_t prefill_slots(int n_tokens, int n_seq, int group) {
 // accesses to different arrays never overlap).
 template <int D>
 struct PrefillLds {
-  static constexpr int kBufBytes = 2 * ChunkGeo<D>::BYTES;  // [stage][K | V], 16-aligned
+  static constexpr int kBufBytes = 2 * ChunkGeo<D, true>::BYTES;  // [stage][K | V], 16-aligned
   char* buf;
   int* tbl;      // kTblCap entries
   int* scan_sh;  // kPW
@@ -89,7 +89,7 @@ struct PairRows {
 // Chunk c of the window [lo, hi): BOTH, for both tokens at once (one read
 // of each K and V^T fragment for the two; the chunk lies below A's limit),
 // else for token B when it sees the chunk.
-template <typename T, int D, bool BOTH>
+template <typename T, int D, bool BOTH, int MASK>
 __device__ __forceinline__ void pair_chunk(PairRows<T, D>& x, int c, int lo, int hi,
                                            const ChunkCtx& cx) {
   const int sb = min(x.lim[1], hi);
@@ -97,13 +97,13 @@ __device__ __forceinline__ void pair_chunk(PairRows<T, D>& x, int c, int lo, int
     floatx4 sacc[2][2];
     const int sh[2] = {min(x.lim[0], hi), sb};
     chunk_scores_sub<T, D, 2, 0, 2>(cx, x.qf, sacc);
-    chunk_update_sub<T, D, 2, 0, 2, true>(c, cx, sh, sacc, x.st);
+    chunk_update_sub<T, D, 2, 0, 2, MASK, true>(c, cx, sh, sacc, x.st);
   } else {
     if (lo + c * kChunk >= sb) return;  // uniform across the wavefront
     floatx4 sacc[1][2];
     const int sh[1] = {sb};
     chunk_scores_sub<T, D, 2, 1, 1>(cx, x.qf, sacc);
-    chunk_update_sub<T, D, 2, 1, 1, true>(c, cx, sh, sacc, x.st);
+    chunk_update_sub<T, D, 2, 1, 1, MASK, true>(c, cx, sh, sacc, x.st);
   }
 }
 
@@ -160,10 +160,10 @@ __device__ __forceinline__ u32x4 new_piece(const AttnArgs& a, int tok, int kvh, 
 }
 
 // Pair `slot` of kv head `kvh` (a workgroup of kPBlock threads).
-template <typename T, int D, int WPT, bool OFF64, bool KV8>
+template <typename T, int D, int WPT, bool OFF64, bool KV8, int MASK = kMaskEnd>
 __device__ __forceinline__ void prefill_pair_body(AttnArgs a, int slot, int kvh,
                                                   const PrefillLds<D>& sm) {
-  using Geo = ChunkGeo<D>;
+  using Geo = ChunkGeo<D, true>;
   constexpr int CPR = Geo::CPR;
   constexpr int PIECES = kChunk * CPR;       // 16-byte pieces of one chunk of K
   constexpr int PER = 2 * PIECES / kPBlock;  // pieces (K and V) per thread
@@ -426,7 +426,7 @@ __device__ __forceinline__ void prefill_pair_body(AttnArgs a, int slot, int kvh,
       cx.kl = kl;
       cx.vl = kl + Geo::KBYTES;
       cx.seg_lo = lo;
-      pair_chunk<T, D, decltype(both)::value>(X, c, lo, hi, cx);
+      pair_chunk<T, D, decltype(both)::value, MASK>(X, c, lo, hi, cx);
       if (lo == 0 && c == 0 && dec) {  // its position has arrived: request the table entry
         const int page = d_pos >> a.bs_shift;
         if (d_pos >= 0 && page < a.max_blk)
