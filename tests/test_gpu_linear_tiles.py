@@ -74,7 +74,7 @@ def test_rope_qkv(m, hq, hkv, d, k):
 
 
 def test_wrappers_take_it_and_gradients_do_not(monkeypatch):
-    x, w = mk(1, 1100, 512), mk(2, 96, 512, std=512 ** -0.5)
+    x, w = mk(1, 1100, 128), mk(2, 96, 128, std=128 ** -0.5)
     calls = []
     real = fused_ops._tiles
     monkeypatch.setattr(fused_ops, "_tiles", lambda *a: calls.append(1) or real(*a))
@@ -99,7 +99,7 @@ def test_slab_counts(k, m, n):
 def test_transformed_calls_stay_with_the_framework():
     """Autocast, forward-mode AD and torch.func see the projection as they see
     F.linear; an x that is the residual itself is read before it is written."""
-    x, w, t = mk(1, 1100, 512), mk(2, 512, 512, std=512 ** -0.5), mk(3, 1100, 512)
+    x, w, t = mk(1, 1100, 128), mk(2, 128, 128, std=128 ** -0.5), mk(3, 1100, 128)
     with torch.no_grad():
         with torch.autocast("cuda", dtype=torch.bfloat16):
             assert fused_ops.linear(x, w).dtype == torch.bfloat16

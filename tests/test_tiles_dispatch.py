@@ -42,6 +42,20 @@ def test_forms_only_the_framework_takes():
     assert not fused_ops._tiles_fit(x[:256], w, None)
 
 
+@pytest.mark.parametrize("rows,n,k,plain,fused", [
+    (257, 96, 32, True, True), (5000, 512, 128, True, True), (300, 513, 128, False, True),
+    (300, 128, 160, False, True), (257, 64, 384, False, True),
+    (512, 512, 512, False, False), (513, 512, 512, False, True), (257, 1024, 416, False, True),
+    (1024, 16384, 544, False, False), (2240, 1024, 1024, False, False),
+    (2305, 1024, 1024, False, True), (8192, 96, 1024, False, False),
+    (2305, 1024, 1056, False, False)])
+def test_sizes_the_tiles_are_faster_at(rows, n, k, plain, fused):
+    """Both sides of each line of the size rule."""
+    x, w = torch.empty(rows, k), torch.empty(n, k)
+    assert fused_ops._tiles_fit(x, w, None, False) == plain
+    assert fused_ops._tiles_fit(x, w, None, True) == fused
+
+
 def test_rotary_tables():
     """A prompt's projection refuses tables of different length, as rope()
     does; the few-row kernels rotate at the positions both tables hold."""

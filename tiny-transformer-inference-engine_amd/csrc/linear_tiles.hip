@@ -4,22 +4,25 @@
 // add, the same arithmetic as the few-row projections' (linear.hip).
 //
 // What bounds it: the fp32 matrix pipe (155 TFLOP/s on this machine), which
-// vector instructions of the same SIMD do not overlap, and on few tiles the
-// last, partly filled round of workgroups. A workgroup owns 64 rows x 64 (or 32)
-// weight rows; k is walked in slabs of 32, loaded in whole 128-byte lines
-// through buffer resources whose scalar offset moves along k (no address
-// arithmetic in the loop), four slabs ahead in registers, staged in two LDS
-// buffers, one barrier a slab. One slab ahead covered 512 to 1024 cycles of
+// vector instructions of the same SIMD do not overlap; at k = 512 it is busy for
+// little more than half the time (gate/up of 2481 rows: 89 TFLOP/s with 97% of
+// the places in five rounds of workgroups filled), the rest is each workgroup's
+// first round trips, its epilogue and the fragment reads. A workgroup owns 64
+// rows x 32 (or 64) weight rows; k is walked in slabs of 32, loaded in whole
+// 128-byte lines through buffer resources whose scalar offset moves along k (no
+// address arithmetic in the loop), four slabs ahead in registers, staged in two
+// LDS buffers, one barrier a slab. One slab ahead covered 512 to 1024 cycles of
 // matrix work against a longer round trip to memory: at 2146 rows x 1024 the
-// three fused forms took 191 us together, now 171; at 512 66 and 60. (Operands
+// three fused forms took 191 us together, then 171; at 512 66 and 60. (Operands
 // loaded straight from memory in matrix layout, without LDS, took 1.5 times as
 // long: sixteen 16-byte pieces of sixteen lines per instruction fill the L1.
 // Slabs of 64, and LDS padding that bounds the workgroups per CU, measured the
 // same.)
-// Measured for a default prefill's layer (2146 rows, 512 wide), GPU time of the
+// Measured for a layer of 2481 rows (eight prompts), 512 wide, GPU time of the
 // library GEMM with its separate element-wise kernel against this one, us:
-// q/k/v + RoPE 33.4 / 19.2, gate/up + SwiGLU 37.7 / 26.4, out + residual 18.3 /
-// 17.2; 4096 rows x 1024 gate/up 134.8 / 138.3 (124 TFLOP/s), all three 311 / 302.
+// q/k/v + RoPE 25.4 / 22.9, gate/up + SwiGLU 46.8 / 29.3, out + residual 19.0 /
+// 18.7; 4096 rows x 1024: 98.9 / 83.0, 134 / 133 (129 TFLOP/s), 73.4 / 70.7. The
+// callers' size rule (serving/fused_ops.py) has the other side.
 #include "mfma_decode_common.h"
 
 namespace pkv {
@@ -239,14 +242,21 @@ __global__ __launch_bounds__(256, 3) void linear_tiles_kernel(TileArgs a) {
   }
 }
 
-// A workgroup owns 64 rows x 64 weight rows, or x 32 where that leaves the last
-// round of workgroups over the CUs emptier (the sum order is the same).
+// A workgroup owns 64 rows x 32 weight rows, or x 64 (the sum order is the same):
+// a round of wide tiles over the CUs takes as long as 1.9 narrow ones, so wide ones
+// run where their rounds cost less, but not below two and a half, where the
+// emptier CUs count more than the fewer operand loads. Wide / narrow, us: 1025
+// rows x 512, k 512 14.2 / 13.0; 1400 x 4096, k 1024 102 / 95; 3000 x 1024, k 1024
+// 55.5 / 60.9; 2481 x 8192, k 1024 328 / 403. Over 330 shapes of 257-8192 rows
+// this costs 0.25% on average against the better one of the two.
 template <int EPI>
 int launch(const TileArgs& a, int64_t weight_rows, hipStream_t stream) {
   const int64_t cus = device_cu_count();
   auto up = [](int64_t x, int64_t y) { return (x + y - 1) / y; };
   const int64_t mt = up(a.m, 64);
-  const bool wide = 2 * up(mt * up(weight_rows, 64), cus) <= up(mt * up(weight_rows, 32), cus);
+  const int64_t wides = mt * up(weight_rows, 64);
+  const bool wide = 2 * wides >= 5 * cus &&
+                    15 * up(wides, cus) <= 8 * up(mt * up(weight_rows, 32), cus);
   const int64_t ny = up(weight_rows, wide ? 64 : 32);
   if (ny > 65535) return fail(PKV_ERR_UNSUPPORTED, "linear_tiles: %lld tiles", (long long)ny);
   const dim3 grid((unsigned)mt, (unsigned)ny);

@@ -191,13 +191,39 @@ def _linear_ok(x2: torch.Tensor, w: torch.Tensor, bias, n_features: int) -> bool
             and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-# fp32 rows pkv_linear_tiles takes from the library GEMM. Sums of a layer's three
-# fused projections, library / tiles, us of GPU time: at k = 512, 300 rows 28.8 /
-# 27.6, 900 40.1 / 39.0, 2146 89 / 63, 4096 111 / 92; at k = 1024, 600 rows 67 / 82,
-# 1300 137 / 121, 2146 222 / 189, 4096 311 / 302; at k = 128, 300 rows 20.2 / 13.7
-TILES_MAX_K = 1024
+# Projections of more than 256 fp32 rows that pkv_linear_tiles takes, by what it
+# was measured to be no slower at than the library GEMM and the element-wise
+# launch of its own (library / tiles, us of GPU time, 257 to 8192 rows):
+#  - without a fused op it saves no launch: k <= TILES_PLAIN_K and up to
+#    TILES_PLAIN_N features (300 x 128, k 128 4.4 / 4.0; but 2481 x 512, k 512
+#    14.9 / 19.0, 257 x 512 6.4 / 8.6);
+#  - fused, k <= TILES_ANY_K: every size (k 128, 2481 rows, gate/up 10.1 / 5.6; at
+#    k 384 1.0 to 1.9 times as fast);
+#  - k <= TILES_SMALL_K: more tiles than half the CUs (2481 rows, k 512: q/k/v
+#    25.4 / 22.9, gate/up 46.8 / 29.3, out 19.0 / 18.7; but q/k/v of 257 rows 9.5 /
+#    10.1);
+#  - k <= TILES_MAX_K: more than TILES_MIN_ROWS rows and four and a half rounds of
+#    tiles over the CUs (k 1024: 2481 rows, gate/up 109 / 87, 8192 rows, out 141 /
+#    135; but 1025 rows, out 27.4 / 30.7, 1600 rows 37.4 / 38.8).
+# Of 1580 shapes inside the lines five are slower by more than 1%, one by 8%.
+TILES_PLAIN_K, TILES_PLAIN_N = 128, 512
+TILES_ANY_K = 384
 TILES_SMALL_K = 512
+TILES_MAX_K = 1024
 TILES_MIN_ROWS = 1024
+CUS = 256
+
+
+def _tiles_faster(rows: int, n: int, k: int, fused: bool) -> bool:
+    """The measured line above; n weight rows in tiles of 64 rows x 32."""
+    if not fused:
+        return k <= TILES_PLAIN_K and n <= TILES_PLAIN_N
+    if k <= TILES_ANY_K:
+        return True
+    tiles = -(-rows // 64) * -(-n // 32)
+    if k <= TILES_SMALL_K:
+        return 2 * tiles > CUS
+    return k <= TILES_MAX_K and rows > TILES_MIN_ROWS and 2 * tiles >= 9 * CUS
 
 
 def _mode_active() -> bool:
@@ -222,28 +248,29 @@ def _transformed(ts) -> bool:
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in ts))
 
 
-def _tiles_fit(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
-    """Whether pkv_linear_tiles takes a projection of these operands. Calls the
+def _tiles_fit(x2: torch.Tensor, w: torch.Tensor, bias, fused: bool = False) -> bool:
+    """Whether pkv_linear_tiles takes a projection of these operands (fused:
+    with an element-wise op in its epilogue). Calls the
     framework has to see stay on its GEMM, and so do forms that only it takes: a
     bias of any other shape than one value per weight row (all the kernel reads),
     a weight that is a vector, sparse or empty, and lazily negated values."""
     ts = (x2, w) if bias is None else (x2, w, bias)
     rows, k = x2.shape
-    return (rows > (LINEAR_MAX_ROWS if k <= TILES_SMALL_K else TILES_MIN_ROWS)
-            and 0 < k <= TILES_MAX_K
+    return (rows > LINEAR_MAX_ROWS and 0 < k <= TILES_MAX_K
             and all(t.dtype == torch.float32 and t.device == x2.device
                     and t.layout is torch.strided for t in ts)
             and not _transformed(ts) and not any(t.is_neg() for t in ts)
             and w.dim() == 2 and w.shape[1] == k and k % 32 == 0
             and 0 < w.shape[0] <= LINEAR_MAX_FEATURES and w.is_contiguous()
+            and _tiles_faster(rows, w.shape[0], k, fused)
             and (bias is None or (bias.shape == w.shape[:1] and bias.is_contiguous()))
             and x2.stride(0) >= k and x2.stride(0) % 4 == 0
             and rows * x2.stride(0) < 1 << 29 and w.numel() < 1 << 29
             and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-def _tiles_ok(x2: torch.Tensor, w: torch.Tensor, bias) -> bool:
-    return x2.is_cuda and _tiles_fit(x2, w, bias)
+def _tiles_ok(x2: torch.Tensor, w: torch.Tensor, bias, fused: bool = False) -> bool:
+    return x2.is_cuda and _tiles_fit(x2, w, bias, fused)
 
 
 def _tiles(out, x2, w, bias, n, epilogue, what):
@@ -284,7 +311,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, b_gate_up: torch.Ten
     x2 = _as_rows(x)
     h = w_gate_up.shape[0] // 2
     if not _linear_ok(x2, w_gate_up, b_gate_up, 2 * h):
-        if w_gate_up.shape[0] == 2 * h and _tiles_ok(x2, w_gate_up, b_gate_up):
+        if w_gate_up.shape[0] == 2 * h and _tiles_ok(x2, w_gate_up, b_gate_up, True):
             out = x.new_empty((x2.shape[0], h))
             _tiles(out, x2, w_gate_up, b_gate_up, h, _native.EPILOGUE_SWIGLU, "linear_swiglu")
             return out.view(*x.shape[:-1], h)
@@ -310,7 +337,7 @@ def linear_rope_qkv(x: torch.Tensor, w_qkv: torch.Tensor, b_qkv: torch.Tensor | 
     T = x2.shape[0]
     nq, nk = hq * d, hkv * d
     few = _linear_ok(x2, w_qkv, b_qkv, nq + 2 * nk)
-    if not few and not (_tiles_ok(x2, w_qkv, b_qkv) and w_qkv.shape[0] == nq + 2 * nk
+    if not few and not (_tiles_ok(x2, w_qkv, b_qkv, True) and w_qkv.shape[0] == nq + 2 * nk
                         and d % 2 == 0):
         qkv = F.linear(x2, w_qkv, b_qkv)
         return rope(qkv[:, :nq], qkv[:, nq:nq + nk], positions, cos, sin, v=qkv[:, nq + nk:],
@@ -376,7 +403,7 @@ def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
     n = weight.shape[0]
     if (not _linear_ok(x2, weight, bias, n) or not resid.is_contiguous()
             or resid.dtype != x.dtype or resid.numel() != x2.shape[0] * n):
-        if (_tiles_resid_fit(resid, x2, n) and _tiles_ok(x2, weight, bias)
+        if (_tiles_resid_fit(resid, x2, n) and _tiles_ok(x2, weight, bias, True)
                 and _apart(resid, x2) and _apart(resid, weight) and _apart(resid, bias)):
             _tiles(resid, x2, weight, bias, n, _native.EPILOGUE_RESIDUAL, "linear_residual_")
             # as add_ does: a graph that saved resid finds it changed
