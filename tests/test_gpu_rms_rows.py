@@ -30,7 +30,8 @@ def norm(x, w, delta, shift):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,dim", [(1, 32), (3, 64), (2, 256), (5, 288), (7, 512), (4, 992),
-                                      (9, 960), (1025, 1024), (3, 1056), (2, 2048), (2, 2080)])
+                                      (9, 960), (1025, 1024), (3, 1056), (2, 2048), (2, 2080),
+                                      (1024, 1056), (1025, 2048)])
 @pytest.mark.parametrize("add", [False, True])
 def test_bits_of_the_row_kernel(dtype, rows, dim, add):
     g = torch.Generator(device=DEV).manual_seed(rows * dim)

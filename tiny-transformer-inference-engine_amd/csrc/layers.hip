@@ -367,9 +367,12 @@ int rms_launch(const RmsArgs& a, int64_t rows, bool vec, hipStream_t stream) {
   constexpr int VV = 16 / sizeof(T);
   const int V = vec ? VV : 1;
   // rows a half wavefront holds in registers; with a residual, few long rows
-  // stay on the row kernel (128 rows x 1024 bf16: 3.2 us there, 3.3 here)
+  // stay on the row kernel (128 rows x 1024 bf16: 3.2 us there, 3.3 here), and
+  // so do 1024 of fp32's longest, which fill the CUs once there (1024 rows x
+  // 2048: 6.5 there, 7.3 here; 1280 rows 8.7 and 8.0)
   const int per = (a.dim / 32 + kNormSplit - 1) / kNormSplit;
-  if (vec && a.dim % 32 == 0 && per <= 8 && (!a.delta || per <= 2 || rows >= 1024)) {
+  const int64_t least = sizeof(T) == 4 && per > 4 ? 1025 : 1024;
+  if (vec && a.dim % 32 == 0 && per <= 8 && (!a.delta || per <= 2 || rows >= least)) {
     const dim3 grid((unsigned)((rows + 1) / 2));
     if (per == 1)
       hipLaunchKernelGGL((rms_rows_kernel<T, 1>), grid, dim3(64), 0, stream, a, (int)rows);
