@@ -31,3 +31,24 @@ def test_null_pointers_and_last_error():
     assert rc == _native.PKV_ERR_INVALID
     with pytest.raises(ValueError, match="null"):
         _native.check(rc, "pkv_rms_norm")
+
+
+@pytest.mark.parametrize("content", [None, b"not a shared object"])
+def test_without_the_module_the_calls_go_through_ctypes(monkeypatch, tmp_path, content):
+    path = tmp_path / "_pkvbind.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_native, "BIND_PATH", str(path))
+    monkeypatch.setattr(_native, "_calls", None)
+    assert _native.calls() is _native.lib()
+    assert _native.calls().pkv_version() >= 1
+
+
+def test_built_without_python_headers(monkeypatch, tmp_path, capsys):
+    import build_native
+    monkeypatch.setattr(build_native, "BIND", str(tmp_path / "_pkvbind.so"))
+    monkeypatch.setattr(build_native, "CXX", "no-such-compiler")
+    (tmp_path / "_pkvbind.so").write_bytes(b"stale")
+    build_native.build_bind()
+    assert "not built" in capsys.readouterr().out
+    assert not (tmp_path / "_pkvbind.so").exists()

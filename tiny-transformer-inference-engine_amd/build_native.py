@@ -80,11 +80,23 @@ def build(jobs: int = 4, verbose: bool = False) -> str:
     tmp = LIB + ".tmp"
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
     os.replace(tmp, LIB)
-    tmp = BIND + ".tmp"
-    _run([CXX, "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall",
-          "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "bind.cpp"), "-o", tmp])
-    os.replace(tmp, BIND)
+    build_bind()
     return LIB
+
+
+def build_bind() -> None:
+    """Compile lib/_pkvbind.so. Without a host compiler or Python's headers there
+    is none, and the wrappers call the library through ctypes."""
+    include = sysconfig.get_paths()["include"]
+    if not shutil.which(CXX) or not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"no {CXX} or no Python.h in {include}: {BIND} is not built")
+        if os.path.exists(BIND):
+            os.remove(BIND)
+        return
+    tmp = BIND + ".tmp"
+    _run([CXX, "-O2", "-fPIC", "-shared", "-std=c++17", "-Wall", "-I", include,
+          os.path.join(CSRC, "bind.cpp"), "-o", tmp])
+    os.replace(tmp, BIND)
 
 
 def clean() -> None:

@@ -4,7 +4,10 @@
 // with the attention's 29 arguments costs about 4 us, as much as the small
 // kernels behind it; these cost under 1. The addresses come from the loaded
 // library (bind()), so both ways reach the same instance. As with ctypes, the
-// interpreter lock is released during the call.
+// interpreter lock is released during the call. Only the stable ABI is used, so
+// one build serves every CPython from 3.10 on; where the module is not there the
+// wrappers call through ctypes (serving/_native.py).
+#define Py_LIMITED_API 0x030A0000
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
