@@ -3,6 +3,7 @@ point, the C argument conversions, and errors reported on the same thread."""
 import pytest
 
 from serving import _native
+from serving.fake_paged_attn import _bound
 
 
 def test_every_entry_point_is_there():
@@ -31,6 +32,16 @@ def test_null_pointers_and_last_error():
     assert rc == _native.PKV_ERR_INVALID
     with pytest.raises(ValueError, match="null"):
         _native.check(rc, "pkv_rms_norm")
+
+
+def test_bounds_fit_the_librarys_int():
+    """A context bound or partition length of any size is accepted (ctypes took
+    its low 32 bits): past 2^30 tokens it bounds nothing."""
+    args = lambda b: (32, 1, 16, 1, 64, 64, 16, b, 0, 2)  # noqa: E731
+    size = _native.calls().pkv_attention_workspace_bytes
+    for b in (1 << 31, (1 << 32) + 5, 1 << 40, 1 << 70):
+        assert size(*args(_bound(b))) == size(*args(0))
+    assert [_bound(b) for b in (-3, 0, 7, 1 << 30, -(1 << 40))] == [-3, 0, 7, 1 << 30, 0]
 
 
 @pytest.mark.parametrize("content", [None, b"not a shared object"])

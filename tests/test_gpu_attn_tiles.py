@@ -14,7 +14,7 @@ import torch
 
 from oracle import paged_ref as ref
 from serving import _native
-from serving.fake_paged_attn import paged_attn_fwd
+from serving.fake_paged_attn import paged_attn_fwd, paged_mqa_decode
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -128,6 +128,15 @@ def test_packed_grid():
     q_lens = [1] * 300
     q_lens[137], q_lens[299] = 70, 33
     check(problem(q_lens, pasts, 8, 1, 64, 16, torch.float32), torch.float32)
+
+
+def test_bounds_past_the_librarys_int():
+    p = problem([1] * 5, [3, 70, 600, 900, 12], 8, 1, 64, 16, torch.float32)
+    args = (p["q"], p["k"], p["v"], p["table"], p["lens"])
+    want = paged_mqa_decode(*args)
+    assert torch.equal(paged_mqa_decode(*args, max_kv_len=1 << 40), want)
+    out = paged_mqa_decode(*args, max_kv_len=(1 << 32) + 5, part_tokens=1 << 40)
+    torch.testing.assert_close(out, want, rtol=1e-5, atol=1e-5)
 
 
 def test_no_visible_key_and_empty_runs():

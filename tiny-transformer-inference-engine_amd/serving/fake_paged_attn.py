@@ -51,6 +51,12 @@ def _check_no_grad(*ts: torch.Tensor) -> None:
             "torch.no_grad() or torch.inference_mode()")
 
 
+def _bound(tokens: int) -> int:
+    """A bound in tokens as the library's int: one past any context it can hold
+    stays no bound at all, whatever its size."""
+    return tokens if -1 << 31 <= tokens <= 1 << 30 else 1 << 30 if tokens > 0 else 0
+
+
 def _launch(q, k_pool, v_pool, block_tables, seq_lens, queryloc, n_seq,
             max_q_len, max_kv_len, scale, causal, out, lse,
             part_tokens: int = 0):
@@ -58,6 +64,7 @@ def _launch(q, k_pool, v_pool, block_tables, seq_lens, queryloc, n_seq,
     nb, bs, hkv, _ = k_pool.shape
     max_blk = block_tables.shape[1] if block_tables.dim() == 2 else 0
     code = _native.kv_code(q.dtype, k_pool.dtype)
+    max_kv_len, part_tokens = _bound(max_kv_len), _bound(part_tokens)
     L = _native.calls()
     ws_bytes = L.pkv_attention_workspace_bytes(
         n_seq, max_q_len, hq, hkv, d, max_blk, bs, max_kv_len, part_tokens, code)
@@ -235,18 +242,19 @@ def paged_attention_append_meta(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     if k.dtype != q.dtype:
         raise TypeError(f"new K/V rows ({k.dtype}) must have the queries' dtype ({q.dtype})")
     code = _native.kv_code(q.dtype, pool.dtype)
+    max_kv_len = _bound(meta.max_kv_len)
     L = _native.calls()
     max_blk = meta.block_tables.shape[1] if meta.block_tables.dim() == 2 else 0
     ws_bytes = L.pkv_attention_workspace_bytes(
         meta.num_seqs, meta.max_q_len, hq, pool.num_kv_heads, d, max_blk, pool.block_size,
-        meta.max_kv_len, 0, code)
+        max_kv_len, 0, code)
     ws = _native.current_workspace().get(q.device, ws_bytes)
     status = pool._status()
     rc = L.pkv_paged_attention_append(
         out.data_ptr(), _native.ptr(lse), q.data_ptr(), kp.data_ptr(), vp.data_ptr(),
         pool.num_blocks, pool.block_size, meta.block_tables.data_ptr() if max_blk else None,
         max_blk, meta.seq_lens.data_ptr(), meta.query_start_loc.data_ptr(), meta.num_seqs, T,
-        meta.max_q_len, meta.max_kv_len, hq, pool.num_kv_heads, d,
+        meta.max_q_len, max_kv_len, hq, pool.num_kv_heads, d,
         float(scale if scale is not None and scale > 0 else 0.0), int(bool(causal)), 0, code,
         k.data_ptr(), v.data_ptr(), meta.start_pos.data_ptr(), _native.ptr(ws), ws_bytes,
         _native.ptr(status), _native.stream_ptr(q.device))
