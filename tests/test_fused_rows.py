@@ -4,9 +4,13 @@ equals the separate weights, the modules' parameters become views of it
 (state-dict keys, shapes and values unchanged; load_state_dict and in-place
 updates reach the fused storage), and a replaced parameter (module.to, a
 new Parameter) triggers a rebuild."""
+import types
+
+import pytest
 import torch
 import torch.nn as nn
 
+from serving import fused_ops
 from serving.fused_ops import FusedRows
 from serving.layers import ModelConfig, SwiGLU
 from serving.paged_mqa import MQA_Paged
@@ -61,3 +65,29 @@ def test_state_dict_round_trip_through_views():
     mlp = SwiGLU(16, 24)
     w, _ = mlp._gate_up.get()
     assert w.shape == (48, 16) and torch.equal(w[24:], mlp.up_proj.weight)
+
+
+class Scaled(torch.nn.Linear):
+    """A subclass whose weight is computed."""
+
+    @property
+    def weight(self):
+        return self._parameters["weight"] * 2
+
+
+def test_module_attr_reads_what_the_module_says():
+    lin = Scaled(4, 4, bias=False)
+    torch.nn.init.ones_(lin._parameters["weight"])
+    assert torch.equal(fused_ops.module_attr(lin, "weight"), lin.weight)
+    assert not torch.equal(lin.weight, lin._parameters["weight"])
+    plain = torch.nn.Linear(4, 4)
+    assert fused_ops.module_attr(plain, "weight") is plain.weight
+    assert fused_ops.module_attr(plain, "bias") is plain.bias
+    assert fused_ops.module_attr(plain, "in_features") == 4
+    del plain.weight
+    plain.weight = torch.ones(4, 4)  # a plain tensor
+    assert fused_ops.module_attr(plain, "weight") is plain.weight
+    norm = types.SimpleNamespace(weight=torch.ones(4), eps=1e-5)  # no Module
+    assert fused_ops.module_attr(norm, "weight") is norm.weight
+    with pytest.raises(AttributeError):
+        fused_ops.module_attr(plain, "nothing")

@@ -526,13 +526,19 @@ def sample_rows(logits: torch.Tensor, temperature: float, top_k: int, top_p: flo
     return ids, status
 
 
-def module_attr(mod: torch.nn.Module, name: str):
-    """mod.<name> for a parameter, buffer or submodule, read from its dict
-    where it is there: nn.Module's own lookup goes through a failed attribute
-    access first (0.25 us each, some thirty a layer)."""
-    for d in (mod._parameters, mod._modules, mod._buffers):
-        if name in d:
-            return d[name]
+# module classes known to have no class attribute in the place of a parameter,
+# buffer or submodule (a subclass may, and is read by its own rules)
+PLAIN_MODULES = {torch.nn.Linear}
+
+
+def module_attr(mod, name: str):
+    """mod.<name> for a parameter, buffer or submodule. Of PLAIN_MODULES it is
+    read from its dict where it is there: nn.Module's own lookup goes through a
+    failed attribute access first (0.25 us each, some thirty a layer)."""
+    if type(mod) in PLAIN_MODULES:
+        for d in (mod._parameters, mod._modules, mod._buffers):
+            if name in d:
+                return d[name]
     return getattr(mod, name)
 
 

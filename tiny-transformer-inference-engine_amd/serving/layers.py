@@ -134,6 +134,9 @@ class SwiGLU(nn.Module):
         return fused_ops.linear_residual_(x, h, attr(down, "weight"), attr(down, "bias"))
 
 
+fused_ops.PLAIN_MODULES.update((RoPE, RMSNorm, SwiGLU))
+
+
 class TokenEmbedding(nn.Module):
     def __init__(self, vocab_size, embed_dim):
         super().__init__()

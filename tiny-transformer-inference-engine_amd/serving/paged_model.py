@@ -35,6 +35,9 @@ class PagedBlock(nn.Module):
         return x + self.mlp(self.mlp_norm(x))
 
 
+fused_ops.PLAIN_MODULES.add(PagedBlock)
+
+
 class PagedTransformer(nn.Module):
     def __init__(self, config, backend="pytorch"):
         super().__init__()

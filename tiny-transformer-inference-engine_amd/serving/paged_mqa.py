@@ -118,3 +118,6 @@ class MQA_Paged(nn.Module):
         proj = attr(self, "out")
         return fused_ops.linear_residual_(x, out.view(T, d_model), attr(proj, "weight"),
                                           attr(proj, "bias"))
+
+
+fused_ops.PLAIN_MODULES.add(MQA_Paged)
