@@ -72,6 +72,8 @@ class Scaled(torch.nn.Linear):
 
     @property
     def weight(self):
+        if "weight" not in self._parameters:
+            raise AttributeError("weight")
         return self._parameters["weight"] * 2
 
 
