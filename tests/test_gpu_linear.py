@@ -248,3 +248,27 @@ def test_fused_norm_past_1024_features_refused_then_composed():
     expect = fused_ops.linear_swiglu(fused_ops.rms_norm(x, nw, 1e-5), w, None)
     torch.cuda.synchronize()
     assert torch.equal(got, expect)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_operands_of_another_shape_or_device(dtype):
+    """What is no [features, k] weight with one bias value per row is F.linear's
+    result or error; the kernels never see it. Tolerance: sums of 64 products of
+    N(0, 1) / 8 values rounded to bf16, 2^-8 of at most 4."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    mk = lambda *s: (torch.randn(s, generator=g, device="cuda") / 8).to(dtype)  # noqa: E731
+    x, w = mk(7, 64), mk(96, 64)
+    tol = dict(rtol=0, atol=1e-5 if dtype == torch.float32 else 2.0 ** -6)
+    with torch.no_grad():
+        for b in (mk(1), mk(1, 96), mk(7, 96)):
+            got = fused_ops.linear(x, w, b)
+            torch.testing.assert_close(got.double(), x.double() @ w.double().t() + b.double(),
+                                       **tol)
+        torch.testing.assert_close(fused_ops.linear(x, w[0]).double(), x.double() @ w[0].double(),
+                                   **tol)
+        for bad in (lambda: fused_ops.linear(x, w, mk(95)), lambda: fused_ops.linear(x, mk(96, 32)),
+                    lambda: fused_ops.linear(x, w.cpu()),
+                    lambda: fused_ops.linear(x, w, mk(96).cpu()),
+                    lambda: fused_ops.linear_residual_(mk(7, 96).cpu(), x, w)):
+            with pytest.raises(RuntimeError):
+                bad()

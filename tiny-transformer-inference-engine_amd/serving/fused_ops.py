@@ -182,13 +182,24 @@ def _as_rows(x: torch.Tensor) -> torch.Tensor:
 
 
 def _linear_ok(x2: torch.Tensor, w: torch.Tensor, bias, n_features: int) -> bool:
-    return (x2.is_cuda and x2.dtype in (torch.bfloat16, torch.float16, torch.float32)
-            and w.dtype == x2.dtype
-            and (bias is None or (bias.dtype == x2.dtype and bias.is_contiguous()))
-            and 0 < x2.shape[0] <= LINEAR_MAX_ROWS and x2.shape[1] % 32 == 0
-            and n_features <= LINEAR_MAX_FEATURES and w.is_contiguous()
-            and (x2.shape[0] == 1 or x2.stride(0) % 8 == 0)
+    rows, k = x2.shape
+    return (x2.is_cuda and 0 < rows <= LINEAR_MAX_ROWS
+            and x2.dtype in (torch.bfloat16, torch.float16, torch.float32)
+            and w.dtype == x2.dtype and w.is_cuda
+            and k % 32 == 0 and n_features <= LINEAR_MAX_FEATURES
+            and _weights_hold(w, n_features, k)
+            # one value per weight row; any other bias is the framework's
+            and (bias is None or (bias.dtype == x2.dtype and bias.is_contiguous()
+                                  and bias.shape == w.shape[:1] and bias.is_cuda))
+            and w.is_contiguous()
+            and (rows == 1 or x2.stride(0) % 8 == 0)
             and x2.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def _weights_hold(w: torch.Tensor, n: int, k: int) -> bool:
+    """Whether w has n rows of k values, as the kernel will read it."""
+    shape = w.shape
+    return len(shape) == 2 and shape[1] == k and shape[0] >= n
 
 
 # Projections of more than 256 fp32 rows that pkv_linear_tiles takes, by what it
@@ -401,7 +412,7 @@ def linear_residual_(resid: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
     x's rows. Returns resid."""
     x2 = _as_rows(x)
     n = weight.shape[0]
-    if (not _linear_ok(x2, weight, bias, n) or not resid.is_contiguous()
+    if (not _linear_ok(x2, weight, bias, n) or not resid.is_contiguous() or not resid.is_cuda
             or resid.dtype != x.dtype or resid.numel() != x2.shape[0] * n):
         if (_tiles_resid_fit(resid, x2, n) and _tiles_ok(x2, weight, bias, True)
                 and _apart(resid, x2) and _apart(resid, weight) and _apart(resid, bias)):
