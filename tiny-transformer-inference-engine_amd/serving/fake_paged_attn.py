@@ -51,10 +51,13 @@ def _check_no_grad(*ts: torch.Tensor) -> None:
             "torch.no_grad() or torch.inference_mode()")
 
 
+MAX_TOKENS = 1 << 30
+
+
 def _bound(tokens: int) -> int:
     """A bound in tokens as the library's int: one past any context it can hold
     stays no bound at all, whatever its size."""
-    return tokens if -1 << 31 <= tokens <= 1 << 30 else 1 << 30 if tokens > 0 else 0
+    return min(tokens, MAX_TOKENS)
 
 
 def _launch(q, k_pool, v_pool, block_tables, seq_lens, queryloc, n_seq,
@@ -64,7 +67,8 @@ def _launch(q, k_pool, v_pool, block_tables, seq_lens, queryloc, n_seq,
     nb, bs, hkv, _ = k_pool.shape
     max_blk = block_tables.shape[1] if block_tables.dim() == 2 else 0
     code = _native.kv_code(q.dtype, k_pool.dtype)
-    max_kv_len, part_tokens = _bound(max_kv_len), _bound(part_tokens)
+    if max_kv_len > MAX_TOKENS or part_tokens > MAX_TOKENS:
+        max_kv_len, part_tokens = _bound(max_kv_len), _bound(part_tokens)
     L = _native.calls()
     ws_bytes = L.pkv_attention_workspace_bytes(
         n_seq, max_q_len, hq, hkv, d, max_blk, bs, max_kv_len, part_tokens, code)
@@ -242,7 +246,9 @@ def paged_attention_append_meta(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     if k.dtype != q.dtype:
         raise TypeError(f"new K/V rows ({k.dtype}) must have the queries' dtype ({q.dtype})")
     code = _native.kv_code(q.dtype, pool.dtype)
-    max_kv_len = _bound(meta.max_kv_len)
+    max_kv_len = meta.max_kv_len
+    if max_kv_len > MAX_TOKENS:
+        max_kv_len = _bound(max_kv_len)
     L = _native.calls()
     max_blk = meta.block_tables.shape[1] if meta.block_tables.dim() == 2 else 0
     ws_bytes = L.pkv_attention_workspace_bytes(

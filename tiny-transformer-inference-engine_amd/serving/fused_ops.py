@@ -144,9 +144,12 @@ def _rope_tables(cos, sin, d, what, equal):
     if cos.dtype != torch.float32 or sin.dtype != torch.float32:
         raise ValueError(f"{what}: cos / sin must be fp32 tables")
     cos2, sin2 = cos.reshape(-1, d // 2).contiguous(), sin.reshape(-1, d // 2).contiguous()
-    if equal and cos2.shape != sin2.shape:
+    shape = cos2.shape
+    if shape == sin2.shape:
+        return cos2, sin2, shape[0]
+    if equal:
         raise ValueError(f"{what}: cos / sin must be tables of equal shape [max_pos, D/2]")
-    return cos2, sin2, min(cos2.shape[0], sin2.shape[0])
+    return cos2, sin2, min(shape[0], sin2.shape[0])
 
 
 def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
@@ -547,9 +550,16 @@ def module_attr(mod, name: str):
     read from its dict where it is there: nn.Module's own lookup goes through a
     failed attribute access first (0.25 us each, some thirty a layer)."""
     if type(mod) in PLAIN_MODULES:
-        for d in (mod._parameters, mod._modules, mod._buffers):
-            if name in d:
-                return d[name]
+        own = mod.__dict__
+        d = own["_parameters"]
+        if name in d:
+            return d[name]
+        d = own["_modules"]
+        if name in d:
+            return d[name]
+        d = own["_buffers"]
+        if name in d:
+            return d[name]
     return getattr(mod, name)
 
 
