@@ -116,9 +116,9 @@ struct Piece {
 // the tile is read through a buffer resource of its own, base its first row
 // and size its rows below kv_hi (0 for a bad table entry), so rows that do not
 // exist read as zeros and every lane's offsets are the same for every tile.
-// The addresses are then scalar work, which matters here: an fp32 matrix
-// instruction and a vector instruction of the same SIMD do not overlap on this
-// machine (238 + 267 us of each, alone, take 501 together), so the per-row
+// The addresses are then scalar work, which matters here: fp32 matrix and vector
+// instructions of one SIMD overlap little on this machine (a loop of both takes
+// 82 to 88% of the sum of the two alone, 1 to 4 wavefronts), so the per-row
 // addresses cost 1.6 us of every 3.1 us step. Smaller blocks keep them.
 template <typename T, int D, int NT, int N, bool WHOLE>
 __device__ __forceinline__ bool tile_chunks(const AttnArgs& a, const int32_t* __restrict__ table,
@@ -555,7 +555,9 @@ __global__ __launch_bounds__(kTBlock, 2) void attn_tiles_kernel(AttnArgs a, int 
 
 // Launch shape, by the number of 32-row tiles that have rows (tiles_max bounds
 // the longest sequence's, n_tokens all of them together; measured at D = 64,
-// fp32, 8 heads, us with the table append's 5):
+// fp32, 8 heads, us with the table append's 5. Other head dims and 16-bit pools
+// take the same lines, which were not measured for them; on both sides of them
+// the kernel is 1.3 to 8 times as fast there as the row kernel):
 //  - up to kHalfWgs of them leave CUs idle: 16-row tiles (one prompt of 500
 //    tokens 12.3 against 17.1);
 //  - up to kOneWgs, the longest first, are balanced best one at a time per CU:

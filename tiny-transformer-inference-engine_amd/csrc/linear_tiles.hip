@@ -4,7 +4,7 @@
 // add, the same arithmetic as the few-row projections' (linear.hip).
 //
 // What bounds it: the fp32 matrix pipe (155 TFLOP/s on this machine), which
-// vector instructions of the same SIMD do not overlap; at k = 512 it is busy for
+// vector instructions of the same SIMD overlap little; at k = 512 it is busy for
 // little more than half the time (gate/up of 2481 rows: 89 TFLOP/s with 97% of
 // the places in five rounds of workgroups filled), the rest is each workgroup's
 // first round trips, its epilogue and the fragment reads. A workgroup owns 64
