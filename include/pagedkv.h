@@ -440,7 +440,8 @@ int pkv_linear_rope_qkv_rmsnorm(void* q_out, void* k_out, void* v_out, const voi
  * Products and sums are fp32; the sum order is fixed and the same for every
  * epilogue of one (m, weight rows, k). dtype must be PKV_DTYPE_F32, k a
  * multiple of 32, x rows, W and out 16-byte aligned, x and W below 2 GiB
- * (PKV_ERR_UNSUPPORTED otherwise). Replaces nn.Linear with the op that
+ * (PKV_ERR_UNSUPPORTED otherwise). out shares no memory with x, W or bias
+ * (other workgroups still read them). Replaces nn.Linear with the op that
  * follows it for a prompt's rows (serving/paged_mqa.py:112-113,
  * models/mlp.py:24-32, serving/paged_model.py:20-29).
  */
